@@ -34,7 +34,7 @@ constexpr int XN = 4096;                     // elements of one bin k_resolve ho
 constexpr unsigned long long M40 = (1ull << 40) - 1;
 
 // ---------------------------------------------------------------------------------------------- block record
-enum : int { RF_CAND = 1, RF_SAMP = 2 };
+enum : int { RF_CAND = 1, RF_SAMP = 2, RF_TOP = 4 };  // RF_TOP: a top-list record (listed_top)
 // Bins of a block are top-down: rel = (c * 64 + 63) - fine bin, so rel 0..63 is the power of two 2^c of the block's
 // best and rel >> 6 = e counts powers of two below it.  Elements with rel >= NBIN weigh nothing in any row.
 struct Rec {
@@ -62,6 +62,62 @@ __device__ inline uint32_t bw_cnt(unsigned long long w) { return (uint32_t)(w >>
 __device__ inline unsigned long long bw_mu(unsigned long long w) { return w & BW_MU; }
 __device__ inline uint32_t bw_off(unsigned long long w) { return (uint32_t)(w >> 51) & 0x7FFu; }
 __device__ inline bool bw_listed(unsigned long long w) { return (w >> 62) & 1ull; }
+
+// ---- top-list records: rows whose top_k is at most TOPK_MAX.  Their kept set lies inside the row's top_k best
+// candidates, so a block records its own best ones (at least top_k of them, or all it has; at most TOPN, unordered) and
+// nothing else: no histogram, no window, no patches.  They fit the record's first 512 bytes, which the resolver reads in
+// its first round of loads: a key and the token's index inside the block, 6 bytes each, in the header's place of the
+// per-power sums.  Measured (k_scan / k_resolve, rocprofv3): 32 bf16 rows, top-k 50, 300 biases 22.0 / 8.9 -> 15.0 / 8.7 us;
+// 80 bf16 verify rows, top-k 50, 46.6 / 22.2 -> 31.0 / 12.7 us; one fp32 row, top-k 20, 10.4 / 14.0 -> 8.4 / 8.0 us.
+// Larger K keeps the general records: its candidates no longer fit one wave, and the bound's overshoot grows with K.
+constexpr int TOPK_MAX = 64;                                  // the kept set fits one wave
+constexpr int TOPN = (int)(HDR_BYTES - 64) / 6;               // 74
+constexpr int TOP_KEYS = 64, TOP_IDS = TOP_KEYS + TOPN * 4;   // byte offsets of u32 okey[TOPN] and u16 local[TOPN]
+static_assert(TOP_IDS + TOPN * 2 <= (int)HDR_BYTES && TOPN >= TOPK_MAX, "top list inside the header");
+// Test flags that ask for rescans, staged draws or separate passes keep the general records.
+__device__ inline bool listed_top(const qws_row& R) {
+  return R.top_k > 0 && R.top_k <= TOPK_MAX && R.temperature > 0.0f && kscale(R.temperature) < INFINITY &&
+         !(R.test_flags & (QWS_TF_RESCAN | QWS_TF_STAGED_DRAW | QWS_TF_SPLIT_SELECT));
+}
+
+// A key that at least `need` of a wave's N keys per lane reach (key(j): the calling lane's j-th), and few more: a
+// bisection between lo (keys below it, as the 0 of an empty place, never count) and the largest key, which stops at the
+// first bound that at most `enough` keys reach.  *n = the keys at or above the returned bound: fewer than `need` only
+// when fewer exist; more than `enough` only when the keys equal to the bound are tied (fewer than `need` above it).
+template <int N, typename T, typename F>
+__device__ __forceinline__ T top_bound(F key, T lo, int need, int enough, int* n) {
+  auto count = [&](T b) {
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < N; j++) c += __popcll(__ballot(key(j) >= b));
+    return c;
+  };
+  T lm = key(0);
+#pragma unroll
+  for (int j = 1; j < N; j++) lm = key(j) > lm ? key(j) : lm;
+  T h, bot;  // past the largest key, and the smallest of the lanes' largest (64 keys or more lie at or above it)
+  if constexpr (sizeof(T) == 8) {
+    h = wave_max_u64(lm) + 1;
+    bot = wave_min_u64(lm);
+  } else {
+    h = wave_max_u32(lm) + 1;
+    bot = ~wave_max_u32(~lm);
+  }
+  if (need <= 64 && bot > lo) lo = bot;
+  int c = count(lo);
+  while (c > enough && h - lo > 1) {  // uniform
+    const T mid = lo + (h - lo) / 2;
+    const int cm = count(mid);
+    if (cm >= need) {
+      lo = mid;
+      c = cm;
+    } else {
+      h = mid;
+    }
+  }
+  *n = c;
+  return lo;
+}
 
 // ---------------------------------------------------------------------------------------------- block searches
 // Wave-level searches over a block's LDS histogram (hist[rel] = count << 40 | mantissa sum) and its per-power sums,
@@ -1218,6 +1274,220 @@ __device__ __forceinline__ void advance_row(const qws_batch& B, const qws_row& R
   }
 }
 
+// ---------------------------------------------------------------------------------------------- top-list rows
+// A row of top-list records (listed_top): its top_k best candidates from the blocks' lists, then min-p, top-p and the
+// draw over them by one wave, one candidate per lane in rank order.  The same definition as the general path: a
+// candidate below the row's weight window weighs nothing and still counts for top-k; min-p, top-k and top-p each keep a
+// prefix of the rank order, so their order does not matter to the kept set.
+// Selection: a bound from the threads' largest entries that at least top_k entries reach (top_bound; the entries are
+// distinct, so it ends), the entries at or above it gathered (about top_k + a few) and ranked by counting.  Latency
+// bound (one workgroup per row): one round of global loads, then LDS round trips; every loop over LDS entries has a
+// fixed length, so that its reads go out together.
+// hdrs: the blocks' records' first 512 bytes; ts: the exp2 table; buf: TOP_BUF bytes.  All threads, uniform arguments;
+// returns the row's token (-1: none) once its outputs are written.  Out of line: inlined into k_resolve it slowed the
+// general rows by its place in the code (C4 resolve 20.5 -> 22.4 us).
+struct TopRow {
+  int row, V, G, K;
+  uint32_t u_draw;
+  float temperature, top_p, min_p;
+  double log2_min_p;
+  int* out_tokens;
+  int* out_info;
+  float* out_probs;
+  RowRes* rres;
+};
+constexpr int TOP_NL1 = 128;               // entries ranked at once
+constexpr int TOP_EPL = (TOPN + 7) / 8;    // entries per thread at most (G > 32: eight threads per block)
+struct TopBuf {
+  uint64_t mxs[NT2];                       // the threads' largest entries, later the reduced list
+  uint64_t lst[64 * TOP_EPL];              // entries at or above the bound (zeros past them, to TOP_NL1)
+  uint32_t rk[4][TOP_NL1];                 // partial ranks
+  uint64_t srt[64];                        // the top_k best in rank order
+  uint64_t w[64];                          // their kept weights (row units)
+  uint64_t part[NWV2][64];                 // partial sums of the kept weights before a candidate in index order
+  uint64_t bound;
+  int cnt, tok;
+};
+static_assert(TOP_NL1 <= NT2 / 4 && TOP_NL1 <= 64 * TOP_EPL && sizeof(TopBuf) <= BIGW * 4, "LDS of resolve_top");
+// Inclusive prefix over lanes of row weights (< 2^59 each: a row of 16 lanes sums to less than 2^63)
+__device__ inline u128 wave_scan_weights(uint64_t v) {
+  v = row16_scan_incl<uint64_t>(v);
+  const uint64_t r0 = readlane<uint64_t>(v, 15), r1 = readlane<uint64_t>(v, 31), r2 = readlane<uint64_t>(v, 47);
+  const int row = lane_id() >> 4;
+  const u128 b1 = r0, b2 = b1 + r1, b3 = b2 + r2;
+  return (u128)v + (row == 0 ? (u128)0 : row == 1 ? b1 : row == 2 ? b2 : b3);
+}
+template <bool VER>
+__device__ __forceinline__ int resolve_top_body(const TopRow& A, const char* hdrs, const float2* ts, TopBuf& L) {
+  constexpr int SLACK = 8;  // entries past top_k accepted by a bound
+  const int tid = threadIdx.x, lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(wave_id());
+  const int K = A.K, G = A.G;
+  // 2^sh threads per block: every thread holds a few entries, spread over as many threads as there are
+  const int sh = G <= 8 ? 6 : G <= 16 ? 5 : G <= 32 ? 4 : 3, g = tid >> sh, j0 = tid & ((1 << sh) - 1);
+  uint64_t c[TOP_EPL], mx = 0;
+  {
+    const char* h = hdrs + (size_t)min(g, G - 1) * HDR_BYTES;
+    const int n = g < G ? min(((const Rec*)h)->n_list, TOPN) : 0;
+#pragma unroll
+    for (int k = 0; k < TOP_EPL; k++) {
+      c[k] = 0;
+      if ((k << sh) >= TOPN) continue;  // uniform
+      const int i = j0 + (k << sh);
+      if (i < n) c[k] = comp(((const uint32_t*)(h + TOP_KEYS))[i], (uint32_t)(g * BLK + ((const uint16_t*)(h + TOP_IDS))[i]));
+      mx = c[k] > mx ? c[k] : mx;
+    }
+  }
+  L.mxs[tid] = mx;
+  if (tid < TOP_NL1) L.lst[tid] = 0ull;
+  if (tid == 0) L.cnt = 0;
+  bar();
+  if (wave == 0) {
+    uint64_t m[NT2 / 64];
+    int cn;
+#pragma unroll
+    for (int j = 0; j < NT2 / 64; j++) m[j] = L.mxs[j * 64 + lane];
+    const uint64_t b = top_bound<NT2 / 64, uint64_t>([&](int j) { return m[j]; }, 1ull, K, min(K + SLACK, 64), &cn);
+    if (lane == 0) L.bound = b;
+  }
+  bar();
+  {
+    const uint64_t b = L.bound;  // at most 64 threads hold entries at or above it
+#pragma unroll
+    for (int k = 0; k < TOP_EPL; k++)
+      if (c[k] >= b) L.lst[atomicAdd(&L.cnt, 1)] = c[k];
+  }
+  bar();
+  int n = __builtin_amdgcn_readfirstlane(L.cnt);
+  const uint64_t* src = L.lst;
+  if (n > TOP_NL1) {  // uniform: the best candidates crowd into few threads' entries
+    if (wave == 0) {
+      auto m = [&](int j) { return j * 64 + lane < n ? L.lst[j * 64 + lane] : 0ull; };
+      int cn, base = 0;
+      const uint64_t b = top_bound<TOP_EPL, uint64_t>(m, 1ull, K, TOP_NL1, &cn);
+      for (int j = 0; j < TOP_EPL; j++) {
+        const uint64_t e = m(j);
+        const unsigned long long bal = __ballot(e >= b);
+        if (e >= b) L.mxs[base + __popcll(bal & ((1ull << lane) - 1ull))] = e;
+        base += __popcll(bal);
+      }
+      for (int i = base + lane; i < TOP_NL1; i += 64) L.mxs[i] = 0ull;
+      if (lane == 0) L.cnt = base;
+    }
+    bar();
+    n = __builtin_amdgcn_readfirstlane(L.cnt);
+    src = L.mxs;
+  }
+  {  // ranks by counting: thread (i, p) counts the larger ones of entries [32 p, 32 p + 32)
+    const int i = tid & (TOP_NL1 - 1), p = tid / TOP_NL1;
+    const uint64_t ci = src[i];
+    uint32_t r = 0;
+    if (TOP_NL1 / 4 * p < n) {  // uniform in the wave
+#pragma unroll
+      for (int j = 0; j < TOP_NL1 / 4; j++) r += src[TOP_NL1 / 4 * p + j] > ci ? 1u : 0u;
+    }
+    L.rk[p][i] = r;
+    bar();
+    if (tid < n) {  // n <= TOP_NL1: p = 0
+      const uint32_t rank = L.rk[0][tid] + L.rk[1][tid] + L.rk[2][tid] + L.rk[3][tid];
+      if (rank < (uint32_t)K) L.srt[rank] = ci;
+    }
+    bar();
+  }
+  // every wave: the row's candidates (top-k applied), one per lane in rank order, weighed and cut by min-p and top-p
+  const int m0 = min(n, K);
+  const uint64_t cc = lane < m0 ? L.srt[lane] : 0ull;
+  const uint32_t idx = comp_idx(cc);
+  const float Ks = kscale(A.temperature);
+  const float t = tval(okey_val(comp_key(cc)), Ks);
+  const float tmax = readlane<float>(t, 0);
+  const int row_top = (tfloor(tmax) >> 10) * FB + (FB - 1);
+  const W ww = weigh(lane < m0 ? t : 0.0f, ts);
+  const int r = row_top - (tfloor(t) >> 4);
+  bool keep = lane < m0 && r < NR;
+  if (A.min_p > 0.0f) keep = keep && t >= (float)((double)(tmax / 1024.0f) + A.log2_min_p) * 1024.0f;
+  uint64_t w = keep ? rw1(ww.mu, r) : 0ull;
+  const u128 incl = wave_scan_weights(w);
+  u128 S2 = readlane<u128>(incl, 63);
+  int m = __popcll(__ballot(w != 0));  // weighted candidates: lanes 0 .. m - 1
+  if (A.top_p < 1.0f) {
+    const u128 thr = mul_shr_ceil(S2, (uint64_t)floor((double)A.top_p * 4294967296.0), 32);
+    if (thr > 0) {
+      m = min(first_lane(w != 0 && thr <= incl), 63) + 1;  // thr <= S2: one lane crosses
+      S2 = readlane<u128>(incl, m - 1);
+      w = lane < m ? w : 0ull;
+    }
+  }
+  // the draw in index order: wave p sums, for each candidate, the kept weights of candidates [8 p, 8 p + 8) with a lower
+  // index (below 2^62), wave 0 adds the eight sums up
+  if (wave * 8 < m) {  // uniform in the wave
+    uint64_t b = 0;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const uint32_t ij = readlane<uint32_t>(idx, wave * 8 + j);
+      const uint64_t wj = readlane<uint64_t>(w, wave * 8 + j);
+      b += ij < idx ? wj : 0ull;
+    }
+    L.part[wave][lane] = b;
+  }
+  bar();
+  if (wave == 0) {
+    const u128 tt = mul_shr_floor(S2, A.u_draw, 24);
+    u128 below = 0;
+#pragma unroll
+    for (int p = 0; p < NWV2; p++)
+      if (p * 8 < m) below += L.part[p][lane];
+    const int l = first_lane(w != 0 && below <= tt && tt < below + w);
+    const int tok = l < 64 ? (int)readlane<uint32_t>(idx, l) : (n == 0 ? 0 : -1);  // no candidate: token 0, as a greedy row's
+    if (A.out_probs && lane < m) {  // k_scan has written zeros
+      const double S2d = (double)(uint64_t)(S2 >> 64) * 18446744073709551616.0 + (double)(uint64_t)S2;
+      A.out_probs[(size_t)A.row * A.V + idx] = (float)((double)w / S2d);
+    }
+    const int rl = readlane<int>(r, max(m - 1, 0));
+    const uint64_t cl = readlane<uint64_t>(cc, max(m - 1, 0));
+    if (lane == 0) {
+      A.out_tokens[A.row] = tok;
+      if (A.out_info) A.out_info[A.row] = n == 0 ? 2 : tok < 0 ? -1 : 0;
+      if (VER) {
+        RowRes o = {};
+        o.kind = n == 0 ? RR_EMPTY : tok < 0 ? RR_FAIL : RR_SAMPLED;
+        o.tok = tok;
+        if (n != 0) {
+          o.s_lo = (unsigned long long)S2;
+          o.s_hi = (unsigned long long)(S2 >> 64);
+          o.cC = cl;  // the kept set: the rank prefix down to its last member
+          o.cR = rl;
+          o.row_top = row_top;
+          o.K = Ks;
+        }
+        A.rres[A.row] = o;
+      }
+      L.tok = tok;
+    }
+  }
+  bar();
+  return __builtin_amdgcn_readfirstlane(L.tok);
+}
+#define QWS_L __attribute__((address_space(3)))
+// The call passes the row's arguments through LDS (an out-of-line function's arguments would arrive in vector registers)
+template <bool VER>
+__device__ __noinline__ int resolve_top(QWS_L const TopRow* a, QWS_L const char* hdrs, QWS_L const float2* ts, QWS_L char* buf) {
+  TopRow A;
+  A.row = __builtin_amdgcn_readfirstlane(a->row);
+  A.V = __builtin_amdgcn_readfirstlane(a->V);
+  A.G = __builtin_amdgcn_readfirstlane(a->G);
+  A.K = __builtin_amdgcn_readfirstlane(a->K);
+  A.u_draw = a->u_draw;
+  A.temperature = a->temperature;
+  A.top_p = a->top_p;
+  A.min_p = a->min_p;
+  A.log2_min_p = a->log2_min_p;
+  A.out_tokens = a->out_tokens;
+  A.out_info = a->out_info;
+  A.out_probs = a->out_probs;
+  A.rres = a->rres;
+  return resolve_top_body<VER>(A, (const char*)hdrs, (const float2*)ts, *(TopBuf*)(char*)buf);
+}
+
 // VER: the rows of a verify call (rres != nullptr)
 template <int DT, bool VER>
 __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, RowRes* rres) {
@@ -1292,6 +1562,14 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
     st.fxn = 0;
   }
   bar();
+  if (listed_top(R)) {  // uniform
+    __shared__ TopRow s_top;
+    if (tid == 0) s_top = TopRow{row, B.V, G, R.top_k, u_draw, R.temperature, R.top_p, R.min_p, R.log2_min_p, B.out_tokens, B.out_info, B.out_probs, rres};
+    bar();
+    const int tk = resolve_top<VER>((QWS_L const TopRow*)&s_top, (QWS_L const char*)s_fb, (QWS_L const float2*)s_ts, (QWS_L char*)s_big);
+    if (!VER && B.advance) advance_row(B, R, row, tk, &s_nt, -1, 0, 0u);
+    return;
+  }
   auto hdr = [&](int g) -> const Rec& { return *(const Rec*)((const char*)s_fb + (size_t)g * HDR_BYTES); };
   if (tid < 64) {  // the row's best: one wave max over the blocks (G <= 64: lane g reads block g)
     uint64_t v = 0;

@@ -22,6 +22,105 @@
 
 namespace qws {
 
+// A block's top-list record (listed_top): its candidates from a bound on that at least top_k of them reach.  The bound
+// comes from the threads' largest elements (lmax: NT1 words of LDS no other wave reads any more): the elements at or
+// above the need-th largest of them are about top_k plus a few, at most 64 threads' elements.  Ties at the bound (equal
+// values in many threads) are taken in index order.  Against the general record (histogram, window, listing) a block
+// costs one comparison per element after the maximum.  area: LDS of the other phases, free once lmax is complete (the
+// barrier after it).  All threads.
+template <int DT, int NT1>
+__device__ __forceinline__ void list_top(const float (&x)[Blk<DT, NT1>::EPT], int lo, int topk, float* lmax, char* area, uint32_t* red, float* s_tv, int* s_tie,
+                                         int* s_n, char* rec) {
+  using BL = Blk<DT, NT1>;
+  constexpr int EPT = BL::EPT, NWV1 = NT1 / 64, SLACK = 8;
+  constexpr int LW_N = 64 * EPT;  // at most 64 threads hold listed elements
+  static_assert(LW_N * 8 <= 18432 && TOPN >= TOPK_MAX, "the list's LDS");
+  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  uint64_t* const LW = (uint64_t*)area;
+  float mloc = -INFINITY;
+#pragma unroll
+  for (int e = 0; e < EPT; e++) mloc = fmaxf(mloc, x[e]);
+  lmax[tid] = mloc;
+  if (tid == 0) *s_n = 0;
+  bar();
+  if (wave == 0) {
+    uint32_t k[NWV1];
+    int c;
+#pragma unroll
+    for (int j = 0; j < NWV1; j++) k[j] = okey(lmax[j * 64 + lane]);
+    const uint32_t b = top_bound<NWV1, uint32_t>([&](int j) { return k[j]; }, KEY_NEGINF + 1u, topk, min(topk + SLACK, 64), &c);
+    if (lane == 0) {
+      const bool tie = c > min(topk + SLACK, 64);
+      *s_tie = tie ? 1 : 0;
+      *s_tv = okey_val(b);
+    }
+  }
+  bar();
+  const bool tie = *s_tie != 0;
+  const float bv = *s_tv;
+  auto take = [&](float v) { return tie ? v > bv : v >= bv; };
+  int nw = 0;
+#pragma unroll
+  for (int e = 0; e < EPT; e++) nw += take(x[e]) ? 1 : 0;
+  const int inc = wave_scan_incl<int>(nw);
+  int wb = 0;
+  if (lane == 63 && inc) wb = atomicAdd(s_n, inc);
+  int off = readlane<int>(wb, 63) + inc - nw;
+#pragma unroll
+  for (int e = 0; e < EPT; e++)
+    if (take(x[e])) LW[off++] = comp(okey(x[e]), (uint32_t)(lo + BL::local(e)));
+  bar();
+  int n = *s_n;
+  if (tie && n < topk) {  // uniform: the first topk - n of the elements equal to the bound, in index order
+    int run = 0;
+    for (int s = 0; s < BL::S; s++) {
+      int ct = 0;
+#pragma unroll
+      for (int e = 0; e < EPT; e++) ct += e / BL::VEC == s && x[e] == bv ? 1 : 0;
+      uint32_t tot;
+      int r = run + (int)block_scan_incl<NWV1, uint32_t>((uint32_t)ct, red, &tot) - ct;
+#pragma unroll
+      for (int e = 0; e < EPT; e++)
+        if (e / BL::VEC == s && x[e] == bv) {
+          if (r < topk - n) LW[n + r] = comp(okey(x[e]), (uint32_t)(lo + BL::local(e)));
+          r++;
+        }
+      run += (int)tot;
+    }
+    n += min(run, topk - n);
+    bar();
+  }
+  uint32_t* const keys = (uint32_t*)(rec + TOP_KEYS);
+  uint16_t* const ids = (uint16_t*)(rec + TOP_IDS);
+  if (n <= TOPN) {  // uniform
+    if (tid < n) {
+      const uint64_t c = LW[tid];
+      keys[tid] = comp_key(c);
+      ids[tid] = (uint16_t)(comp_idx(c) - (uint32_t)lo);
+    }
+  } else if (wave == 0) {  // the best elements crowd into few threads: the list cut to at most TOPN
+    auto k = [&](int j) { return j * 64 + lane < n ? LW[j * 64 + lane] : 0ull; };
+    int c, base = 0;
+    const uint64_t b = top_bound<EPT, uint64_t>(k, 1ull, topk, TOPN, &c);
+    for (int j = 0; j < EPT; j++) {
+      const uint64_t e = k(j);
+      const unsigned long long bal = __ballot(e >= b);
+      if (e >= b) {
+        const int p = base + __popcll(bal & ((1ull << lane) - 1ull));
+        keys[p] = comp_key(e);
+        ids[p] = (uint16_t)(comp_idx(e) - (uint32_t)lo);
+      }
+      base += __popcll(bal);
+    }
+    n = base;
+  }
+  if (tid == 0) {  // a lane of the wave that cut the list
+    Rec* H = (Rec*)rec;
+    H->flags = n > 0 ? RF_CAND | RF_TOP : RF_TOP;
+    H->n_list = n;
+  }
+}
+
 // ---------------------------------------------------------------------------------------------- k_scan
 template <int DT, int NT1>
 __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 != NT1S ? 4 : DT == QWS_DTYPE_BF16 ? 8 : 6))) k_scan(qws_batch B, int G, char* ws, VerifyIO VIO) {
@@ -109,7 +208,8 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
   // goes to the next; the small grids' 1,024-thread workgroups all run at once)
   float blb = -INFINITY;
   const bool stop_on = R.n_stop > 0 && R.min_tokens > R.ngen + R.n_drafts;
-  const bool lbrow = NT1 == NT1S && R.proc_on && R.n_bias > 0 && R.repetition == 1.0f && R.presence == 0.0f && R.frequency == 0.0f &&
+  const bool toprow = listed_top(R);
+  const bool lbrow = NT1 == NT1S && !toprow && R.proc_on && R.n_bias > 0 && R.repetition == 1.0f && R.presence == 0.0f && R.frequency == 0.0f &&
                      R.temperature > 0.0f && (!stop_on || R.n_stop <= 16);
   if (lbrow) {  // uniform
     for (int j = tid; j < R.n_bias; j += NT1) {
@@ -137,6 +237,12 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
       const int i = lo + BL::local(e);
       if (i < hi) B.out_probs[(size_t)row * B.V + i] = 0.0f;
     }
+  }
+  if (toprow) {  // uniform
+    // the touched-token list's LDS is read last before load_processed's last barrier: free for the threads' maxima
+    static_assert(LCAP2 * 4 >= NT1 * 4 && O_LIST >= 18432, "the maxima beside the list's area");
+    list_top<DT, NT1>(x, lo, R.top_k, (float*)(s_lds + O_LIST), s_lds, (uint32_t*)s_redf, (float*)&s_win[0], &s_win[1], &s_nl, rec);
+    return;
   }
   // ---- best candidate: the largest value, lowest index
   float mloc = -INFINITY;
