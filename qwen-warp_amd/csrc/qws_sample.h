@@ -22,12 +22,14 @@ constexpr int NT2 = 512, NWV2 = NT2 / 64;    // k_resolve workgroup
 // k_resolve's grid: workgroup i takes row (i mod 8) * ceil(B / 8) + i / 8, the row k_scan ran on workgroup i's XCD
 inline unsigned resolve_grid(int B) { return (unsigned)(NXCD * ((B + NXCD - 1) / NXCD)); }
 constexpr int CAP = 1024;                    // elements a block may list
-// top-p: fine bins listed at most on either side of the block's own boundary (as many as the list holds): a flat
-// block's boundary is close to the row's, a peaked block's (its top CTOP elements carry a real share of its mass) far
-// less so: its window widens to MARGIN_NEAR, then, when that fits whole, to MARGIN, trimmed to the list's capacity from
-// below first (a row's cut tends to lie above a peaked block's own boundary, and bins above it hold fewer elements)
-constexpr int MARGIN_FLAT = 6, MARGIN_NEAR = 31, MARGIN = 100;
-constexpr int CTOP = 256;                    // elements of a block's top bins listed beside a window further down
+// top-p windows.  A flat block's own boundary is close to the row's: MARGIN_FLAT fine bins on either side.  A peaked
+// block (its top CTOP elements carry a quarter of its mass) lists one range of as many bins as the list holds, from
+// MARGIN_NEAR bins below its boundary upwards (from its top when that fits): the row's boundary tends to lie above a
+// block's own, since the outliers of other blocks add mass at the top.  In a CPU model of the windows over rows of 31
+// blocks (top-p 0.95), against a top part of 256 elements beside 100 bins around the boundary: N(0, 2.5) logits with 32
+// tokens 8 higher, missed blocks per row 6.6 / 3.3 / 8.0 -> 0.1 / 0 / 3.7 at T 0.8 / 0.9 / 1.0; N(0, 3) 0.7 -> 0.
+constexpr int MARGIN_FLAT = 6, MARGIN_NEAR = 31;
+constexpr int CTOP = 256;
 constexpr int MAXG = 64;                     // blocks per row (V <= 524,288)
 constexpr int NR = NBIN;                     // row bins with a nonzero weight (row-relative, 0 = the top)
 constexpr int XN = 4096;                     // elements of one bin k_resolve holds in LDS
@@ -41,9 +43,9 @@ struct Rec {
   uint32_t max_key, max_idx;     // best candidate (okey, lowest index); KEY_NEGINF: none
   int c, flags;                  // power of two of the best; RF_*
   int nbw;                       // bins written: rel 0 .. nbw - 1 (every bin a cut of any row can fall in)
-  int w0, w1, wa, ea;            // listed bins: rel in [w0, w1] with rel <= wa or rel >= ea (none when w0 > w1)
-  int n_list, n_patch, pad0;     // listed elements; processed touched tokens recorded (-1: more than TCAP)
-  uint32_t pad1[4];
+  int w0, w1;                    // listed bins: rel in [w0, w1] (none when w0 > w1)
+  int n_list, n_patch;           // listed elements; processed touched tokens recorded (-1: more than TCAP)
+  uint32_t pad[7];
   uint32_t ecnt[NEXP];           // candidates of power of two e = rel >> 6
   unsigned long long emu[NEXP];  // their summed mantissas (< 2^37)
 };
@@ -152,18 +154,6 @@ __device__ inline int blk_cross_cnt(const unsigned long long* hist, const uint32
   const int f = first_lane(fi >= tgt);
   return p * FB + min(f, 63);
 }
-// first bin whose inclusive cumulative approximate mass reaches tgt (NBIN when none)
-__device__ inline int blk_cross_mass(const unsigned long long* hist, const unsigned long long* emu, float tgt) {
-  const int lane = lane_id();
-  const float pm = lane < NEXP ? ldexpf((float)emu[lane], -lane) : 0.0f;
-  const float inc = wave_scan_incl<float>(pm);
-  const int p = first_lane(lane < NEXP && inc >= tgt);
-  if (p >= NEXP) return NBIN;
-  const float base = readlane<float>(inc - pm, p);
-  const float fi = wave_scan_incl<float>(ldexpf((float)(hist[p * FB + lane] & M40), -p)) + base;
-  const int f = first_lane(fi >= tgt);
-  return p * FB + min(f, 63);
-}
 
 // ---------------------------------------------------------------------------------------------- k_resolve
 // One workgroup per row.  Global loads come in few parallel rounds (the headers; the fine bins of one power of two of
@@ -179,7 +169,7 @@ struct BI {                      // a block as the resolver uses it
   int dn;                        // N - c (row powers of two above the block's top one); -1: nothing of it weighs in the row
   int gcnt, goff, gsrc, gofs;    // the bin being gathered: the block's count, list offset, source (0 none, 1 list, 2 rescan),
                                  // first slot in the gathered list
-  int w0, w1, wa, ea;            // the block's listed bins (its record header's window)
+  int w0, w1;                    // the block's listed bins (its record header's window)
   int n_list, wcnt;              // its listed elements; its candidates inside the row's weight window
 };
 
@@ -1586,8 +1576,6 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
       b.gcnt = b.goff = b.gsrc = b.gofs = 0;
       b.w0 = H.w0;
       b.w1 = H.w1;
-      b.wa = H.wa;
-      b.ea = H.ea;
       b.n_list = H.n_list;
       b.wcnt = 0;
       s_bi[tid] = b;
@@ -1727,7 +1715,7 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
         const int cb = cR - FB * b.dn;  // the cut's bin among the block's own
         if (cb >= 0) {
           const unsigned long long wd = s_fb[lane * FB + (cR & 63)];
-          ok = cb < b.nbw && b.w0 == 0 && cb <= b.w1 && (cb <= b.wa || b.ea == b.wa + 1) && bw_listed(wd);
+          ok = cb < b.nbw && b.w0 == 0 && cb <= b.w1 && bw_listed(wd);
           cnt = ok ? (int)(bw_off(wd) + bw_cnt(wd)) : 0;
         }
       }
@@ -1906,10 +1894,10 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
         if (cR == NR) {
           // no cut: the block's candidates inside the weight window, a top-down prefix of its bins as the (gap-free) list
           // is, lie whole in the list iff they are no more than the list holds
-          if ((b.wa >= b.w1 || b.ea == b.wa + 1) && b.wcnt <= b.n_list) nlist = b.n_list;
+          if (b.wcnt <= b.n_list) nlist = b.n_list;
         } else if (st.fpow == (cR >> 6)) {  // the cut's power is the staged one
           const int cb = cR - FB * b.dn;    // the cut's bin among the block's own
-          if (cb >= 0 && cb <= b.w1 && (cb <= b.wa || b.ea == b.wa + 1)) {  // bins 0 .. cb all listed
+          if (cb >= 0 && cb <= b.w1) {  // bins 0 .. cb all listed
             const unsigned long long wd = s_fb[gs * FB + (cR & 63)];
             if (bw_listed(wd)) nlist = (int)(bw_off(wd) + bw_cnt(wd));
           }

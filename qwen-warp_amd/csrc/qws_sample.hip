@@ -290,8 +290,6 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
       H->nbw = 0;
       H->w0 = 1;
       H->w1 = 0;
-      H->wa = -1;
-      H->ea = 0;
       H->n_list = 0;
       H->n_patch = n_patch;
     }
@@ -394,7 +392,7 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
       floor_r = min(floor_r, blk_cross_cnt(hist, s_ecnt, kk));
     }
     floor_r = min(floor_r, r1);
-    int w0 = 1, w1 = 0, wa = -1, ea = 0;
+    int w0 = 1, w1 = 0;
     // power-level inclusive prefixes: counts (exact) and approximate masses (relative to the block's top power); when
     // floor_r is the last occupied bin the block's totals cover it
     const uint32_t pcn = lane < NEXP ? s_ecnt[lane] : 0u;
@@ -402,26 +400,6 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
     const uint32_t icn = wave_scan_incl<uint32_t>(pcn);
     const float ims = wave_scan_incl<float>(pms);
     const bool at_last = floor_r == r1;
-    // inclusive prefix of the bin counts over [a, b] into P (the list cursors' space, written only after the window
-    // is chosen; wave 0 alone writes and reads it); returns b - a + 1
-    uint32_t* P = cursor;
-    auto prefix_counts = [&](int a, int b) {
-      constexpr int PR = (2 * MARGIN + 64) / 64;  // rounds of 64 bins for the widest span (2 MARGIN + 1 bins)
-      const int span = b - a + 1;
-      uint32_t cv[PR];  // every count read before the scans
-#pragma unroll
-      for (int r = 0; r < PR; r++) cv[r] = r * 64 + lane < span ? (uint32_t)(hist[a + r * 64 + lane] >> 40) : 0u;
-      uint32_t carry = 0;
-#pragma unroll
-      for (int r = 0; r < PR; r++) {
-        if (r * 64 < span) {  // uniform
-          const uint32_t inc = wave_scan_incl<uint32_t>(cv[r]) + carry;
-          if (r * 64 + lane < span) P[r * 64 + lane] = inc;
-          carry = readlane<uint32_t>(inc, 63);
-        }
-      }
-      return span;
-    };
     bool slots_done = false;  // the list slots already written (a flat top-p window, from the shrink's prefix)
     uint32_t slots_n = 0;
     if (topk || topp || minp) {
@@ -429,14 +407,12 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
       if (nf <= (uint32_t)CAP) {  // the whole top set
         w0 = 0;
         w1 = floor_r;
-        wa = floor_r;
-        ea = floor_r + 1;
       } else {
-        int a = 0, b = -1, tp = -1;
-        uint32_t budget = (uint32_t)CAP;
+        int b = floor_r;
+        bool flat = false;
         if (topp) {
-          // the block's own top-p boundary bp (mass crossing) and the bin t1 before its (CTOP + 1)-th candidate, both
-          // from the power-level prefixes above and one fine-bin scan each (independent: issued together)
+          // the block's own top-p boundary bp (mass crossing) and the power of its (CTOP + 1)-th candidate, both from
+          // the power-level prefixes above and one fine-bin scan each (independent: issued together)
           const float mf = at_last ? readlane<float>(ims, NEXP - 1) : blk_mass_to(hist, s_emu, floor_r);
           const float tm = R.top_p * mf;
           const uint32_t tc = (uint32_t)CTOP + 1u;  // < nf: pC < NEXP
@@ -445,169 +421,91 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
           const float bmP = pP > 0 && pP < NEXP ? readlane<float>(ims, pP - 1) : 0.0f;
           const float fmP = wave_scan_incl<float>(ldexpf((float)(hP & M40), -pP)) + bmP;
           const int bp = min(pP < NEXP ? pP * FB + min(first_lane(fmP >= tm), 63) : NBIN, floor_r);
-          // a peaked block also lists its top bins (up to CTOP elements) when they carry a real share of its mass:
-          // the row's boundary then lies near the top for a block far below the row's best.  Those elements lie in the
-          // powers through pC, so when the (approximate) mass through pC is below the share, the block is not peaked
-          // and the fine scans of pC are skipped.
-          const bool maybe_peaked = readlane<float>(ims, pC) >= 0.25f * mf;
-          unsigned long long hC = 0ull;
-          if (maybe_peaked) hC = hist[pC * FB + lane];  // uniform
-          const uint32_t bcC = pC > 0 ? readlane<uint32_t>(icn, pC - 1) : 0u;
-          const float bmC = pC > 0 ? readlane<float>(ims, pC - 1) : 0.0f;
-          const uint32_t fcC = maybe_peaked ? wave_scan_incl<uint32_t>((uint32_t)(hC >> 40)) + bcC : 0u;
-          const float fmC = maybe_peaked ? wave_scan_incl<float>(ldexpf((float)(hC & M40), -pC)) + bmC : 0.0f;
-          const int fC = min(first_lane(fcC >= tc), 63);
-          const int tu = pC * FB + fC - 1, t1 = min(tu, floor_r);
-          if (maybe_peaked && t1 >= r0) {
-            // mass and count up to t1: when t1 = tu, inside power pC from its fine scans (fC > 0) or all of the powers
-            // above pC (fC = 0); a floor below tu takes the general sums
-            const bool fast = tu <= floor_r, inC = fC > 0;
-            const float m1 = fast ? (inC ? readlane<float>(fmC, fC - 1) : bmC) : blk_mass_to(hist, s_emu, t1);
-            if (m1 >= 0.25f * mf) {
-              tp = t1;
-              budget -= fast ? (inC ? readlane<uint32_t>(fcC, fC - 1) : bcC) : blk_cnt_to(hist, s_ecnt, tp);
-            }
+          // peaked: the top CTOP elements carry a quarter of the mass.  They lie in the powers through pC, so when the
+          // (approximate) mass through pC is below that, the block is flat and the fine scans of pC are skipped.
+          flat = true;
+          if (readlane<float>(ims, pC) >= 0.25f * mf) {  // uniform
+            const unsigned long long hC = hist[pC * FB + lane];
+            const uint32_t bcC = pC > 0 ? readlane<uint32_t>(icn, pC - 1) : 0u;
+            const float bmC = pC > 0 ? readlane<float>(ims, pC - 1) : 0.0f;
+            const uint32_t fcC = wave_scan_incl<uint32_t>((uint32_t)(hC >> 40)) + bcC;
+            const float fmC = wave_scan_incl<float>(ldexpf((float)(hC & M40), -pC)) + bmC;
+            const int fC = min(first_lane(fcC >= tc), 63);
+            flat = (fC > 0 ? readlane<float>(fmC, fC - 1) : bmC) < 0.25f * mf;
           }
-          // shrink to the budget, keeping the block's own boundary near the middle: bins leave one at a time from the
-          // side farther from bp (the b side on a tie), so the longer side first loses its excess, then the sides
-          // alternate starting with b (removed_b(k, D): the bins gone from the b side after k removals, k - that from
-          // the a side, D = how many the b side loses first; returned by value, as references into the caller's locals
-          // would put them in scratch).  First within MARGIN_FLAT or (peaked) MARGIN_NEAR of bp (one lane per k, the
-          // counts' prefix in registers); for a peaked block whose window fits whole, within MARGIN of bp, the b side
-          // (below bp) first trimmed to MARGIN_NEAR (the prefix in LDS).  The first window that fits the budget (or is
-          // empty) is kept.
-          auto removed_b = [](int k, int D) -> int {
-            if (D >= 0) return k <= D ? k : D + (k - D + 1) / 2;
-            return k - (k <= -D ? k : -D + (k + D) / 2);
-          };
-          const int mn = tp >= 0 ? MARGIN_NEAR : MARGIN_FLAT;
-          a = max(0, bp - mn);
-          b = min(floor_r, bp + mn);
-          int kk;
-          {
-            const int span = b - a + 1;  // <= 2 MARGIN_NEAR + 1 < 64
-            static_assert(2 * MARGIN_NEAR + 1 < 64 && MARGIN_FLAT <= MARGIN_NEAR, "one lane per k");
-            const uint32_t pre = wave_scan_incl<uint32_t>(lane < span ? (uint32_t)(hist[a + lane] >> 40) : 0u);
-            const int k = min(lane, span), kb = removed_b(k, (b - bp) - (bp - a)), ka = k - kb;
-            const int wa = a + ka, wb = b - kb;
-            const uint32_t hi = (uint32_t)__shfl((int)pre, max(wb - a, 0)), lo0 = (uint32_t)__shfl((int)pre, max(ka - 1, 0));
-            const uint32_t n = wa > wb ? 0u : hi - (ka > 0 ? lo0 : 0u);
-            kk = first_lane(lane <= span && n <= budget);
-            const int a0 = a;
-            a = readlane<int>(wa, kk);
-            b = readlane<int>(wb, kk);
-            if (tp < 0 && a <= b) {  // uniform: a flat window [a, b] is listed whole, its slots from the prefix above
-              const uint32_t pb = (uint32_t)__shfl((int)pre, max(lane - 1, 0)), c0 = a > a0 ? readlane<uint32_t>(pre, a - a0 - 1) : 0u;
-              const int r = a0 + lane;
-              if (r >= a && r <= b) cursor[r] = (lane > 0 ? pb : 0u) - c0;
-              slots_done = true;
-              slots_n = readlane<uint32_t>(pre, b - a0) - c0;
-            }
-          }
-          if (tp >= 0 && kk == 0 && (bp - MARGIN_NEAR > 0 || bp + MARGIN_NEAR < floor_r)) {
-            a = max(0, bp - MARGIN);
-            b = min(floor_r, bp + MARGIN);
-            const int span = prefix_counts(a, b);
-            const int D = max(b - bp - MARGIN_NEAR, 0);
-            // the elements left after k removals never grow with k, and k = span empties the window: the first k that
-            // fits, by two rounds of one k per lane (every s-th k, then the s - 1 before the first that fits)
-            auto fits = [&](int k) {
-              const int kb = removed_b(k, D), ka = k - kb;
-              const int wa = a + ka, wb = b - kb;
-              const uint32_t n = wa > wb ? 0u : P[max(wb - a, 0)] - (ka > 0 ? P[ka - 1] : 0u);
-              return n <= budget;
+          if (flat) {
+            // within MARGIN_FLAT of bp, shrunk to the list's capacity one bin at a time from the side farther from bp
+            // (the b side on a tie): the longer side first loses its excess, then the sides alternate starting with b
+            // (removed_b(k, D): the bins gone from the b side after k removals, k - that from the a side, D = how many
+            // the b side loses first; returned by value, as references into the caller's locals would put them in
+            // scratch).  One lane per k, the counts' prefix in registers; the first window that fits (or is empty).
+            auto removed_b = [](int k, int D) -> int {
+              if (D >= 0) return k <= D ? k : D + (k - D + 1) / 2;
+              return k - (k <= -D ? k : -D + (k + D) / 2);
             };
-            const int s = (span + 62) / 63;  // 63 s >= span: lane 63 tries k = span
-            const int k1 = min(lane * s, span);
-            const int f1 = min(first_lane(fits(k1)), 63);
-            if (f1 == 0) {
-              kk = 0;
-            } else {
-              const int kp = readlane<int>(k1, f1 - 1), kn = readlane<int>(k1, f1);  // fits(kn), not fits(kp)
-              const int k2 = kp + 1 + lane;
-              kk = kp + 1 + min(first_lane(k2 <= kn && fits(k2)), kn - kp - 1);
+            const int a0 = max(0, bp - MARGIN_FLAT), b0 = min(floor_r, bp + MARGIN_FLAT);
+            const int span = b0 - a0 + 1;
+            static_assert(2 * MARGIN_FLAT + 1 < 64, "one lane per k");
+            const uint32_t pre = wave_scan_incl<uint32_t>(lane < span ? (uint32_t)(hist[a0 + lane] >> 40) : 0u);
+            const int k = min(lane, span), kb = removed_b(k, (b0 - bp) - (bp - a0)), ka = k - kb;
+            const int wa = a0 + ka, wb = b0 - kb;
+            const uint32_t hi = (uint32_t)__shfl((int)pre, max(wb - a0, 0)), lo0 = (uint32_t)__shfl((int)pre, max(ka - 1, 0));
+            const uint32_t n = wa > wb ? 0u : hi - (ka > 0 ? lo0 : 0u);
+            const int kk = first_lane(lane <= span && n <= (uint32_t)CAP);
+            const int wl = readlane<int>(wa, kk), wr = readlane<int>(wb, kk);
+            if (wl <= wr) {  // uniform: its slots from the prefix above
+              w0 = wl;
+              w1 = wr;
+              const uint32_t pb = (uint32_t)__shfl((int)pre, max(lane - 1, 0)), c0 = wl > a0 ? readlane<uint32_t>(pre, wl - a0 - 1) : 0u;
+              const int r = a0 + lane;
+              if (r >= wl && r <= wr) cursor[r] = (lane > 0 ? pb : 0u) - c0;
+              slots_done = true;
+              slots_n = readlane<uint32_t>(pre, wr - a0) - c0;
             }
-            const int kb = removed_b(kk, D), ka = kk - kb;
-            a += ka;
-            b -= kb;
-          }
-        } else {  // a min-p / top-k floor with more than CAP tokens above it: the bins just above the floor
-          // the first bin from which the bins down to the floor hold at most CAP elements (b + 1: none), first within
-          // 2 MARGIN_NEAR bins of the floor, then, when those all fit, within 2 MARGIN
-          b = floor_r;
-          a = max(0, floor_r - 2 * MARGIN_NEAR);
-          int kk;
-          {
-            const int span = b - a + 1;  // < 64
-            const uint32_t pre = wave_scan_incl<uint32_t>(lane < span ? (uint32_t)(hist[a + lane] >> 40) : 0u);
-            const uint32_t tot = readlane<uint32_t>(pre, 63), lo0 = (uint32_t)__shfl((int)pre, max(lane - 1, 0));
-            const uint32_t n = tot - (lane > 0 ? lo0 : 0u);
-            kk = first_lane(lane <= span && (lane == span || n <= (uint32_t)CAP));
-            a += kk;
-          }
-          if (kk == 0 && a > 0) {
-            a = max(0, floor_r - 2 * MARGIN);
-            const int span = prefix_counts(a, b);
-            const uint32_t tot = P[span - 1];
-            kk = span;
-            for (int k0 = 0; k0 < span; k0 += 64) {  // uniform
-              const int k = k0 + lane;
-              const uint32_t n = k < span ? tot - (k > 0 ? P[k - 1] : 0u) : 0u;
-              const int f = first_lane(k < span && n <= (uint32_t)CAP);
-              if (f < 64) {
-                kk = k0 + f;
-                break;
-              }
-            }
-            a += kk;
+          } else {
+            b = min(floor_r, bp + MARGIN_NEAR);
           }
         }
-        if (tp >= 0) {  // the top part [0, tp], and [a, b] below it (one range when they touch)
-          w0 = 0;
-          w1 = max(b, tp);
-          wa = a <= tp + 1 ? w1 : tp;
-          ea = a <= tp + 1 ? w1 + 1 : a;
-        } else if (a <= b) {
-          w0 = a;
-          w1 = b;
-          wa = b;
-          ea = b + 1;
+        if (!flat) {  // uniform
+          // one range of as many bins as the list holds: from the top when that reaches b (or a min-p floor, which lies
+          // higher in the row than in most of its blocks), else the bins ending at b
+          const uint32_t nb = b == floor_r ? nf : blk_cnt_to(hist, s_ecnt, b);
+          if (minp || nb <= (uint32_t)CAP) {
+            w0 = 0;
+            w1 = min(blk_cross_cnt(hist, s_ecnt, (uint32_t)CAP + 1u) - 1, floor_r);
+          } else {
+            w0 = blk_cross_cnt(hist, s_ecnt, nb - (uint32_t)CAP) + 1;
+            w1 = b;
+          }
         }
       }
     }
-    // list slots: a prefix of the listed bins' counts, in rel order, over the listed ranges [w0, wa] and [ea, w1] (the
-    // bins between them are not listed and get no slot: a peaked block's gap can span hundreds of bins)
-    // (four rounds of 64 bins per step, their counts read together: a peaked block's top range can span ~500 bins)
+    // list slots: a prefix of the listed bins' counts, in rel order (four rounds of 64 bins per step, their counts read
+    // together: a peaked block's range can span hundreds of bins)
     uint32_t base = slots_n;
-    for (int part = 0; part < (slots_done ? 0 : 2); part++) {  // uniform
-      const int lo_r = part == 0 ? w0 : max(ea, w0), hi_r = part == 0 ? min(wa, w1) : w1;
-      for (int r0c = lo_r; r0c <= hi_r; r0c += 256) {
-        uint32_t cn[4];
+    for (int r0c = w0; r0c <= (slots_done ? -1 : w1); r0c += 256) {  // uniform
+      uint32_t cn[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) cn[j] = r0c + 64 * j + lane <= hi_r ? (uint32_t)(hist[r0c + 64 * j + lane] >> 40) : 0u;
+      for (int j = 0; j < 4; j++) cn[j] = r0c + 64 * j + lane <= w1 ? (uint32_t)(hist[r0c + 64 * j + lane] >> 40) : 0u;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          if (r0c + 64 * j > hi_r) break;  // uniform
-          const int r = r0c + 64 * j + lane;
-          const uint32_t inc = wave_scan_incl<uint32_t>(cn[j]);
-          if (r <= hi_r) cursor[r] = base + inc - cn[j];
-          base += readlane<uint32_t>(inc, 63);
-        }
+      for (int j = 0; j < 4; j++) {
+        if (r0c + 64 * j > w1) break;  // uniform
+        const int r = r0c + 64 * j + lane;
+        const uint32_t inc = wave_scan_incl<uint32_t>(cn[j]);
+        if (r <= w1) cursor[r] = base + inc - cn[j];
+        base += readlane<uint32_t>(inc, 63);
       }
     }
     if (lane == 0) {
       s_win[0] = w0;
       s_win[1] = w1;
-      s_win[2] = wa;
-      s_win[3] = ea;
       s_win[4] = (int)base;
       s_win[5] = min(r1, hard) + 1;
       s_nl = 0;
     }
   }
   bar();
-  const int w0 = s_win[0], w1 = s_win[1], wa = s_win[2], ea = s_win[3], nbw = s_win[5];
-  auto listed = [&](int r) { return r >= w0 && r <= w1 && (r <= wa || r >= ea); };
+  const int w0 = s_win[0], w1 = s_win[1], nbw = s_win[5];
   // ---- the record: header, per-power sums, bin words (with the list slots of the listed bins)
   if (tid == 0) {
     H->max_key = okey(M);
@@ -617,8 +515,6 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
     H->nbw = nbw;
     H->w0 = w0;
     H->w1 = w1;
-    H->wa = wa;
-    H->ea = ea;
     H->n_list = s_win[4];
     H->n_patch = n_patch;
   }
@@ -631,7 +527,7 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
   for (int r = tid; r < nbw; r += NT1) {
     const unsigned long long h = hist[r];
     unsigned long long wd = (h & M40) | ((h >> 40) << 37);
-    if (listed(r)) wd |= (1ull << 62) | ((unsigned long long)cursor[r] << 51);
+    if (r >= w0 && r <= w1) wd |= (1ull << 62) | ((unsigned long long)cursor[r] << 51);
     BW[r] = wd;
   }
   if (w0 <= w1) {
@@ -646,48 +542,19 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
       return readlane<int>(wb, 63) + inc - nw;
     };
     auto rel_of = [&](int e) { return (rp[e >> 1] >> ((e & 1) * 16)) & 0xFFFFu; };  // bin, >= NBIN outside
-    if (ea == wa + 1 || wa >= w1) {
-      // one range: one test per element (bins below w0 wrap past span; those >= NBIN lie past it), counted, then
-      // every element written without a branch, the unlisted ones into the lane's dummy slot (never read)
-      const uint32_t span = (uint32_t)(w1 - w0), b0u = (uint32_t)w0;
-      int nw = 0;
+    // one test per element (bins below w0 wrap past span; those >= NBIN lie past it), counted, then every element
+    // written without a branch, the unlisted ones into the lane's dummy slot (never read)
+    const uint32_t span = (uint32_t)(w1 - w0), b0u = (uint32_t)w0;
+    int nw = 0;
 #pragma unroll
-      for (int e = 0; e < EPT; e++) nw += rel_of(e) - b0u <= span ? 1 : 0;
-      uint64_t* dst = LW + wave_base(nw);
-      uint64_t* dummy = (uint64_t*)(dummy_slots + lane);
+    for (int e = 0; e < EPT; e++) nw += rel_of(e) - b0u <= span ? 1 : 0;
+    uint64_t* dst = LW + wave_base(nw);
+    uint64_t* dummy = (uint64_t*)(dummy_slots + lane);
 #pragma unroll
-      for (int e = 0; e < EPT; e++) {
-        const bool l = rel_of(e) - b0u <= span;
-        *(l ? dst : dummy) = ((uint64_t)__float_as_uint(x[e]) << 32) | (uint32_t)BL::local(e);
-        dst += l ? 1 : 0;
-      }
-    } else if constexpr (DT == QWS_DTYPE_F32) {
-      // two ranges, [w0, wa] and [ea, w1] (the second empty when ea > w1): the same two passes with two tests
-      // (fp32 only: in the bf16 kernel, at 64 VGPRs, they spill)
-      const uint32_t s1 = (uint32_t)(wa - w0), b1 = (uint32_t)w0;
-      const uint32_t s2 = ea <= w1 ? (uint32_t)(w1 - ea) : 0u, b2 = ea <= w1 ? (uint32_t)ea : 0xFFFFFFFFu;  // bins < 2^16
-      auto in2 = [&](uint32_t r) { return r - b1 <= s1 || r - b2 <= s2; };
-      int nw = 0;
-#pragma unroll
-      for (int e = 0; e < EPT; e++) nw += in2(rel_of(e)) ? 1 : 0;
-      uint64_t* dst = LW + wave_base(nw);
-      uint64_t* dummy = (uint64_t*)(dummy_slots + lane);
-#pragma unroll
-      for (int e = 0; e < EPT; e++) {
-        const bool l = in2(rel_of(e));
-        *(l ? dst : dummy) = ((uint64_t)__float_as_uint(x[e]) << 32) | (uint32_t)BL::local(e);
-        dst += l ? 1 : 0;
-      }
-    } else {
-      uint32_t lm = 0;  // bit e: element e is listed
-#pragma unroll
-      for (int e = 0; e < EPT; e++) {
-        lm |= listed((int)rel_of(e)) ? 1u << e : 0u;  // bins >= NBIN lie past w1
-      }
-      int off = wave_base(__popc(lm));
-#pragma unroll
-      for (int e = 0; e < EPT; e++)
-        if ((lm >> e) & 1u) LW[off++] = ((uint64_t)__float_as_uint(x[e]) << 32) | (uint32_t)BL::local(e);
+    for (int e = 0; e < EPT; e++) {
+      const bool l = rel_of(e) - b0u <= span;
+      *(l ? dst : dummy) = ((uint64_t)__float_as_uint(x[e]) << 32) | (uint32_t)BL::local(e);
+      dst += l ? 1 : 0;
     }
     bar();
     const int nl = s_nl;
