@@ -178,8 +178,8 @@ struct RS {                      // row state (LDS)
   int fpow;                      // row power of two whose fine bins are staged (-1: none)
   int gbin, gn, gl, gstaged;     // the gathered bin: row bin, elements, listed ones, held in LDS
   int gres;                      // blocks of the gathered bin rescanned (their window missed it)
-  unsigned long long gfast;      // bit g: block g is rescanned straight from its raw logits (no mask, no processed tokens)
-  unsigned long long gslow;      // bit g: block g is rescanned through the staged block (mask or processed tokens)
+  unsigned long long gfast;      // bit g: block g is rescanned straight from its raw logits and patches
+  unsigned long long gslow;      // bit g: block g is rescanned through the staged block (more processed tokens than patches)
   int rescans;                   // blocks rescanned because their window missed a bin
   float K;
   unsigned long long best;
@@ -547,7 +547,7 @@ __device__ __forceinline__ void gather(const RL& L, const qws_batch& B, const qw
       b.goff = (int)bw_off(w);
       b.gsrc = cn == 0 ? 0 : ((bw_listed(w) && !(R.test_flags & QWS_TF_RESCAN)) ? 1 : 2);
       ln = b.gsrc == 1 ? cn : 0u;
-      fr = b.gsrc == 2 && !R.mask_mode && b.n_patch == 0 ? cn : 0u;
+      fr = b.gsrc == 2 && b.n_patch >= 0 ? cn : 0u;
       nres = b.gsrc == 2 ? 1 : 0;
     }
     const uint32_t linc = wave_scan_incl<uint32_t>(ln), finc = wave_scan_incl<uint32_t>(fr);
@@ -607,13 +607,33 @@ __device__ __forceinline__ void gather(const RL& L, const qws_batch& B, const qw
     bar();
     using BL = Blk<DT, NT2>;
     {
-      // blocks without processed tokens or a mask: their raw logits are their values, read straight into registers,
-      // RB blocks at once (all their loads in flight together); only the bin's elements are weighed, each placed at its
-      // block's next slot
+      // blocks whose processed tokens are all recorded as patches: raw logits straight into registers, RB blocks at once
+      // (all their loads in flight together); only the bin's elements are weighed, each placed at its block's next
+      // slot.  Masked and processed tokens are marked in a bitmap per block (in L.big) that the raw values found are
+      // tested against, and the patches' values are tested themselves.  (Through the staged block, one at a time, a
+      // block costs ~5 us: rows that missed 20-30 blocks took 75-150 us in all.)
       constexpr int RB = 8;  // the resolver runs one workgroup per CU: registers for eight blocks of loads in flight
+      constexpr int BW32 = BLK / 32;
+      static_assert(RB * BW32 <= BIGW && NT2 == 2 * BW32 && TCAP == 2 * NT2, "bitmap words and patches per thread");
+      uint32_t* const bm = L.big;
+      const uint32_t flip = R.mask_mode == QWS_MASK_ALLOWED ? 0xFFFFFFFFu : 0u;
+      const unsigned* const mrow = B.masks + (R.mask_mode ? (size_t)R.mask_row * (size_t)B.mask_words : 0);
       const int qb = st.row_top - rb;  // the bin's floor(t) >> 4
       const float K = st.K;
       const XRange xr = bin_xrange(qb, K);
+      auto place = [&](BI& b, int g, int local, float v) {  // the value v of block g's token, when it lies in the bin
+        const float t = tval(v, K);
+        if (v == v && v != -INFINITY && (tfloor(t) >> 4) == qb) {  // NaN counts as -inf
+          const int p = b.gofs + atomicAdd(&b.goff, 1);
+          const uint64_t c = comp(okey(v), (uint32_t)(g * BLK + local));
+          mn = c < mn ? c : mn;
+          mx = c > mx ? c : mx;
+          if (p < XG) {  // always: the bin words count these elements
+            L.ec[p] = c;
+            L.em[p] = weigh(t, L.ts).mu;
+          }
+        }
+      };
       unsigned long long fm = st.gfast;  // uniform
       while (fm) {
         int gb[RB];
@@ -635,6 +655,43 @@ __device__ __forceinline__ void gather(const RL& L, const qws_batch& B, const qw
             BL::load_raw(B, row, gk * BLK, min(B.V, gk * BLK + BLK), x[k]);  // -inf past V; NaN tested below
           }
         }
+        bool marks = R.mask_mode != 0;  // uniform
+#pragma unroll
+        for (int k = 0; k < RB; k++) marks = marks || (gb[k] >= 0 && L.bi[gb[k]].n_patch > 0);
+        if (marks) {
+          uint2 pv[RB][2];
+#pragma unroll
+          for (int k = 0; k < RB; k++) {
+            const int np = gb[k] >= 0 ? L.bi[gb[k]].n_patch : 0;
+            const QWS_G unsigned long long* PT = gmem((const unsigned long long*)(rec_of(ws, G, row, max(gb[k], 0)) + PATCH_OFF));
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+              const unsigned long long w = tid + i * NT2 < np ? PT[tid + i * NT2] : 0xFFFFFFFFull;  // local ~0: none
+              pv[k][i] = make_uint2((uint32_t)w, (uint32_t)(w >> 32));
+            }
+          }
+          const int hw = tid / BW32, wi = tid % BW32;
+          uint32_t mv[RB / 2];
+#pragma unroll
+          for (int k = 0; k < RB / 2; k++) {
+            const int gk = hw ? gb[2 * k + 1] : gb[2 * k], i = gk * BW32 + wi;
+            mv[k] = R.mask_mode && gk >= 0 && i * 32 < B.V ? gmem(mrow)[i] ^ flip : 0u;
+          }
+          bar();  // the bitmaps of the batch before are read no more
+#pragma unroll
+          for (int k = 0; k < RB / 2; k++) bm[(2 * k + hw) * BW32 + wi] = mv[k];
+          bar();
+#pragma unroll
+          for (int k = 0; k < RB; k++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+              if (pv[k][i].x != 0xFFFFFFFFu) {
+                atomicOr(&bm[k * BW32 + (pv[k][i].x >> 5)], 1u << (pv[k][i].x & 31));
+                const float v = __uint_as_float(pv[k][i].y);
+                if (xr.maybe(v)) place(L.bi[gb[k]], gb[k], (int)pv[k][i].x, v);
+              }
+          bar();
+        }
 #pragma unroll
         for (int k = 0; k < RB; k++) {
           if (gb[k] < 0) continue;
@@ -643,17 +700,9 @@ __device__ __forceinline__ void gather(const RL& L, const qws_batch& B, const qw
           for (int e = 0; e < BL::EPT; e++) {
             const float v = x[k][e];
             if (!xr.maybe(v)) continue;  // NaN fails it too
-            const float t = tval(v, K);
-            if (v == v && v != -INFINITY && (tfloor(t) >> 4) == qb) {  // NaN counts as -inf
-              const int p = b.gofs + atomicAdd(&b.goff, 1);
-              const uint64_t c = comp(okey(v), (uint32_t)(gb[k] * BLK + BL::local(e)));
-              mn = c < mn ? c : mn;
-              mx = c > mx ? c : mx;
-              if (p < XG) {  // always: the bin words count these elements
-                L.ec[p] = c;
-                L.em[p] = weigh(t, L.ts).mu;
-              }
-            }
+            const int l = BL::local(e);
+            if (marks && ((bm[k * BW32 + (l >> 5)] >> (l & 31)) & 1u)) continue;
+            place(b, gb[k], l, v);
           }
         }
       }
@@ -1647,7 +1696,15 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
   if (R.min_p > 0.0f) {
     const float tcut = (float)((double)(tmax / 1024.0f) + R.log2_min_p) * 1024.0f;
     const int rc = row_top - (tfloor(tcut) >> 4);
-    if (rc < NR) {
+    bool need = rc < NR;
+    if (need && R.top_k > 0) {  // uniform: top_k candidates in the bins above the min-p cut's: the top-k cut decides
+      stage_power(L, ws, row, rc >> 6);
+      u128 mass_unused;
+      unsigned long long above;
+      before_bin(L, rc, &mass_unused, &above);
+      need = above < (unsigned long long)R.top_k;
+    }
+    if (need) {
       stage_power(L, ws, row, rc >> 6);
       gather<DT, VER>(L, BB, RR, ws, row, rc);
       // kept: t >= tcut, a prefix of the bin in comp order
