@@ -5,9 +5,12 @@ otherwise -- there is no CPU fallback.  The error convention is the reference's 
 a nonzero status raises RuntimeError.
 """
 import ctypes as C
+import importlib.machinery
+import importlib.util
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libqws.so"
+HOSTPACK_PATH = LIB_PATH.with_name("_qws_hostpack.so")
 
 OK, ERR_INVALID, ERR_NOT_SUPPORTED = 0, 1, 801
 NOALLOC_SCRATCH_BYTES = 16 << 20  # include/qws.h QWS_NOALLOC_SCRATCH_BYTES
@@ -142,6 +145,22 @@ def load(path=None):
     if path is None:
         _LIB = lib
     return lib
+
+
+_HOSTPACK = None
+
+
+def hostpack():
+    """The host packing module (csrc/qws_hostpack.cpp), loaded once."""
+    global _HOSTPACK
+    if _HOSTPACK is None:
+        if not HOSTPACK_PATH.exists():
+            raise RuntimeError(f"_qws_hostpack.so not built ({HOSTPACK_PATH}); run python qwen-warp_amd/build.py")
+        loader = importlib.machinery.ExtensionFileLoader("_qws_hostpack", str(HOSTPACK_PATH))
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_qws_hostpack", loader))
+        loader.exec_module(mod)
+        _HOSTPACK = mod
+    return _HOSTPACK
 
 
 def check(err, what=""):

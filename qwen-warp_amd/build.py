@@ -1,4 +1,5 @@
-"""Builds libqws.so (HIP, gfx950) in-tree: qwen-warp_amd/lib/libqws.so.
+"""Builds libqws.so (HIP, gfx950) in-tree, qwen-warp_amd/lib/libqws.so, and beside it the host packing module
+_qws_hostpack.so (C++ over the CPython API, for the interpreter that runs the build).
 
   python qwen-warp_amd/build.py
 
@@ -10,6 +11,7 @@ floating-point operation one IEEE rounding, as the CPU definition), no fast-math
 import os
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
@@ -19,6 +21,8 @@ ROOT = PKG.parent
 SRC = [PKG / "csrc" / "qws_sample.hip", PKG / "csrc" / "qws_verify.hip", PKG / "csrc" / "qws_state.hip", PKG / "csrc" / "qws_pld.hip", PKG / "csrc" / "qws_head.hip",
        PKG / "csrc" / "qws_hooks.hip"]
 OUT = PKG / "lib" / "libqws.so"
+HOST_SRC, HOST_OUT = PKG / "csrc" / "qws_hostpack.cpp", PKG / "lib" / "_qws_hostpack.so"
+CXX = os.environ.get("CXX", "g++")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", f"-I{ROOT / 'include'}"]
@@ -28,7 +32,7 @@ def _run(cmd):
     r = subprocess.run(cmd, capture_output=True, text=True)
     errs = "\n".join(l for l in (r.stdout + r.stderr).splitlines() if "packed-fp32-ops" not in l)
     if r.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({r.returncode}): {' '.join(map(str, cmd))}\n{errs}")
+        raise RuntimeError(f"compiler failed ({r.returncode}): {' '.join(map(str, cmd))}\n{errs}")
 
 
 def build(verbose: bool = False) -> Path:
@@ -44,6 +48,9 @@ def build(verbose: bool = False) -> Path:
         tmp = OUT.with_suffix(".so.tmp")
         _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)])
         os.replace(tmp, OUT)
+        tmp = HOST_OUT.with_suffix(".so.tmp")
+        _run([CXX, "-O2", "-std=c++17", "-fPIC", "-shared", f"-I{sysconfig.get_paths()['include']}", str(HOST_SRC), "-o", str(tmp)])
+        os.replace(tmp, HOST_OUT)
     return OUT
 
 

@@ -18,6 +18,7 @@ from __future__ import annotations
 import ctypes as C
 import math
 import random
+import struct
 from dataclasses import dataclass, field
 from typing import Optional, Sequence
 
@@ -213,9 +214,19 @@ def draft_row(temperature=0.0, top_k=20, top_p=1.0, draft_sample=1, draft_temper
     return RowSpec(temperature=t, top_k=k, top_p=p, min_p=0.0, seed=seed, position=position, stream=ST_DRAFT + int(j), row_key=row_key)
 
 
+_NO_IDS = np.zeros(0, np.int64)
+_NO_IDS.flags.writeable = False
+
+
 def _ids(ids, V, name) -> np.ndarray:
     """Token ids (a list, tuple, set, dict keys, numpy array or tensor) as one int64 array in iteration order, converted
     once; ValidationError unless every id is an integer in [0, V) (a float or bool array is refused, not truncated)."""
+    if type(ids) is list or type(ids) is tuple:  # exact ints in range: one native pass
+        if not ids:
+            return _NO_IDS
+        a = np.empty(len(ids), np.int64)
+        if _lib.hostpack().ids(ids, V, a) == len(ids):
+            return a
     if isinstance(ids, torch.Tensor):
         if ids.numel() and (ids.dtype == torch.bool or ids.dtype.is_floating_point or ids.dtype.is_complex):  # empty: any dtype
             raise ValidationError(f"{name}: token ids must be integers, got a {ids.dtype} tensor", name)
@@ -250,20 +261,30 @@ def penalties_need_state(r: "RowSpec") -> bool:
     return r.procs_on() and int(r.state_slot) < 0 and (r.repetition != 1.0 or r.presence != 0.0 or r.frequency != 0.0)
 
 
+_ROW = struct.Struct("=f i f f d Q 3I i 3f 17i")  # include/qws.h qws_row, field by field
+_BATCH = struct.Struct("@P 3i q 7P i 4P P 2i")             # include/qws.h qws_batch
+assert _ROW.size == C.sizeof(Row) and _BATCH.size == C.sizeof(Batch)
+
+
 class PackedBatch:
     """Rows packed into device arrays (CSR histories, bias, stop ids, masks) and the qws_batch struct.  Rows with a
     state_slot take their prompt set and generated counts from `state` (a ProcState) instead of a CSR history:
     their prompt / gen lists are not packed, and ngen (for min_tokens) is r.ngen, else len(r.gen)."""
 
-    def __init__(self, rows: Sequence[RowSpec], V: int, device, state: Optional["ProcState"] = None):
+    def __init__(self, rows: Sequence[RowSpec], V: int, device, state: Optional["ProcState"] = None, ordered: bool = False):
+        """ordered=True: the device copy is ordered on the current stream but not waited for, for a caller that runs the
+        batch on that stream only (the calls that pack their own rows); otherwise it is complete on return, so that the
+        batch may run on any stream."""
         self.B, self.V = len(rows), V
         self.state = state
         if state is not None and state.V != V:
             raise ValidationError(f"the ProcState holds V={state.V}, the batch V={V}", "state")
         W = (V + 31) // 32
-        hr, hist, drafts, bids, bvals, stops, masks = [], [], [], [], [], [], []
-        nh = nd = 0  # entries of hist and drafts so far
-        for r in rows:
+        hist, drafts, bids, bvals, stops, masks = [], [], [], [], [], []
+        nh = nd = nb_all = ns = 0  # entries of hist, drafts, bids and stops so far
+        rowb = bytearray(C.sizeof(Row) * self.B)
+        slots, dup_slot, need_state = set(), False, False
+        for k, r in enumerate(rows):
             if not (r.repetition > 0.0) or r.min_tokens < 0:
                 raise ValidationError("repetition must be > 0 and min_tokens >= 0", "repetition_penalty", r.repetition)
             if not (0.0 < r.top_p <= 1.0) or not (0.0 <= r.min_p <= 1.0):
@@ -273,84 +294,102 @@ class PackedBatch:
             allowed = _ids(r.allowed, V, "allowed") if r.allowed is not None else None
             if allowed is not None and allowed.size == 0:
                 allowed = None  # an empty allowed list masks nothing
-            bkeys = _ids((r.bias or {}).keys(), V, "logit_bias")
+            bkeys = _ids(list(r.bias), V, "logit_bias") if r.bias else _NO_IDS
             ng = len(gen) if r.ngen is None else int(r.ngen)
             st = int(r.state_slot)
             if st >= 0 and (state is None or st >= state.slots):
                 raise ValidationError(f"state_slot {st} needs a ProcState with more than {st} slots", "state_slot", st)
             if len(gen) + len(rdrafts) > HIST_MAX:
                 raise ValidationError(f"history longer than {HIST_MAX} tokens", "history", len(gen) + len(rdrafts))
-            nb = len(r.bias or {})
+            nb = len(bkeys)
             if nb > BIAS_MAX_ROW:
                 raise ValidationError(f"logit_bias has {nb} entries, at most {BIAS_MAX_ROW} per row", "logit_bias", nb)
-            row = Row()
             on = r.procs_on()
-            row.temperature, row.top_k, row.top_p, row.min_p = r.temperature, r.top_k, r.top_p, r.min_p
-            row.log2_min_p = math.log2(float(np.float32(r.min_p))) if r.min_p > 0 else 0.0
-            row.seed, row.position, row.stream, row.row_key = int(r.seed) & (2 ** 64 - 1), r.position & 0xFFFFFFFF, r.stream, r.row_key & 0xFFFFFFFF
-            row.proc_on = int(on)
-            row.presence, row.frequency, row.repetition, row.min_tokens, row.ngen = r.presence, r.frequency, r.repetition, r.min_tokens, ng
-            row.test_flags, row.draw_word = r.test_flags, r.draw_word
-            row.state_slot = st if st >= 0 else -1
+            if st >= 0:
+                dup_slot = dup_slot or st in slots
+                slots.add(st)
+            elif on and penalties_need_state(r):
+                need_state = True
+            lists = [0] * 8  # hist_off, n_prompt, n_gen, draft_off, n_drafts, bias_off, n_bias, stop_off
+            n_stop = mask_mode = mask_row = 0
             if on:
-                row.hist_off = nh
+                lists[0] = nh
                 if st < 0:
-                    row.n_prompt, row.n_gen = len(prompt), len(gen)
+                    lists[1], lists[2] = len(prompt), len(gen)
                     hist += [prompt, gen]
                     nh += len(prompt) + len(gen)
-                row.draft_off, row.n_drafts = nd, len(rdrafts)
+                lists[3], lists[4] = nd, len(rdrafts)
                 drafts.append(rdrafts)
                 nd += len(rdrafts)
-                row.bias_off, row.n_bias = len(bids), nb
-                bids += bkeys.tolist()
-                bvals += [float(v) for v in (r.bias or {}).values()]
-                row.stop_off, row.n_stop = len(stops), len(rstop)
-                stops += rstop.tolist()
+                lists[5], lists[6] = nb_all, nb
+                if nb:
+                    bids.append(bkeys)
+                    bvals += [float(v) for v in r.bias.values()]
+                    nb_all += nb
+                lists[7], n_stop = ns, len(rstop)
+                if n_stop:
+                    stops.append(rstop)
+                    ns += n_stop
                 if allowed is not None:
                     m = np.zeros(W, np.uint32)
                     a = allowed
                     np.bitwise_or.at(m, a >> 5, (np.uint32(1) << (a & 31).astype(np.uint32)))
                     if r.banned is not None:
                         m &= ~np.asarray(r.banned, dtype=np.uint32)[:W]
-                    row.mask_mode, row.mask_row = MASK_ALLOWED, len(masks)
+                    mask_mode, mask_row = MASK_ALLOWED, len(masks)
                     masks.append(m)
                 elif r.banned is not None:
-                    row.mask_mode, row.mask_row = MASK_BANNED, len(masks)
+                    mask_mode, mask_row = MASK_BANNED, len(masks)
                     masks.append(np.asarray(r.banned, dtype=np.uint32)[:W])
-            hr.append(row)
+                if mask_mode and masks[mask_row].shape != (W,):
+                    raise ValidationError(f"a mask must hold {W} words", "banned")
+            vals = (r.temperature, r.top_k, r.top_p, r.min_p, math.log2(float(np.float32(r.min_p))) if r.min_p > 0 else 0.0, int(r.seed) & (2 ** 64 - 1),
+                    r.position & 0xFFFFFFFF, r.stream, r.row_key & 0xFFFFFFFF, int(on), r.presence, r.frequency, r.repetition, r.min_tokens, ng, *lists, n_stop,
+                    mask_mode, mask_row, r.test_flags, r.draw_word, st if st >= 0 else -1, 0)
+            try:
+                _ROW.pack_into(rowb, k * _ROW.size, *vals)
+            except (struct.error, OverflowError):  # a value past its field: the conversions of the ctypes structure
+                row = Row()
+                for (name, _), v in zip(Row._fields_, vals):
+                    setattr(row, name, v)
+                rowb[k * _ROW.size:(k + 1) * _ROW.size] = bytes(row)
         dev = torch.device(device)
 
-        def arr(a, dt):  # one element at least, so that every array has a device address
-            return np.concatenate(a).astype(dt) if a and isinstance(a[0], np.ndarray) else (np.asarray(a, dtype=dt) if len(a) else np.zeros(1, dt))
-
-        # every array in one host buffer (256-byte aligned parts) and one host-to-device copy; the device arrays are
-        # views of it
-        parts = [np.frombuffer((Row * self.B)(*hr), dtype=np.uint8), arr(hist, np.int32), arr(drafts, np.int32), arr(bids, np.int32),
-                 arr(bvals, np.float32), arr(stops, np.int32), np.stack(masks).astype(np.uint32) if masks else np.zeros(0, np.uint32)]
+        # every array in one host buffer (256-byte aligned parts, one element at least, so that every array has a device
+        # address) and one host-to-device copy; the device arrays are views of it
+        sizes = [len(rowb), 4 * max(nh, 1), 4 * max(nd, 1), 4 * max(nb_all, 1), 4 * max(nb_all, 1), 4 * max(ns, 1), 4 * W * len(masks)]
         offs, n = [], 0
-        for a in parts:
+        for z in sizes:
             offs.append(n)
-            n += (a.nbytes + 255) & ~255
-        buf = np.zeros(max(n, 256), np.uint8)
-        for a, o in zip(parts, offs):
-            buf[o:o + a.nbytes] = a.reshape(-1).view(np.uint8)
-        self.dev_buf = torch.from_numpy(buf).to(dev)
-        view = [self.dev_buf[o:o + a.nbytes] for a, o in zip(parts, offs)]
+            n += (z + 255) & ~255
+        ordered = ordered and dev.type == "cuda" and not torch.cuda.is_current_stream_capturing()
+        host = torch.empty(n, dtype=torch.uint8, pin_memory=True) if ordered else torch.zeros(n, dtype=torch.uint8)
+        buf = host.numpy()
+        buf[:len(rowb)] = np.frombuffer(rowb, np.uint8)
+        for o, arrs in zip(offs[1:], (hist, drafts, bids, None, stops, masks)):
+            for a in arrs or ():
+                if len(a):
+                    buf[o:o + 4 * len(a)].view(np.uint32 if arrs is masks else np.int32)[:] = a
+                    o += 4 * len(a)
+        if nb_all:
+            buf[offs[4]:offs[4] + 4 * nb_all].view(np.float32)[:] = bvals
+        self.dev_buf = host.to(dev, non_blocking=ordered)
+        view = [self.dev_buf[o:o + z] for o, z in zip(offs, sizes)]
         self.rows_t = view[0]
         self.hist_t, self.drafts_t, self.bids_t = view[1].view(torch.int32), view[2].view(torch.int32), view[3].view(torch.int32)
         self.bvals_t, self.stops_t = view[4].view(torch.float32), view[5].view(torch.int32)
         self.masks_t = view[6].view(torch.int32).reshape(len(masks), W) if masks else None
         self.W = W
-        self.host_rows = hr
+        self.host_rows = (Row * self.B).from_buffer_copy(rowb)
         self.specs = list(rows)
+        self._dup_slot, self._need_state = dup_slot, need_state
 
     def check_advance(self):
         """The rows may take their decode step on the device (qws_batch.advance, qws_finish_rows): distinct state slots,
-        and penalties that count generated tokens kept in a state slot (penalties_need_state)."""
-        slots = [r.state_slot for r in self.host_rows if r.state_slot >= 0]
-        if len(set(slots)) != len(slots):
+        and penalties that count generated tokens kept in a state slot (penalties_need_state), as they were packed."""
+        if self._dup_slot:
             raise ValidationError("advance needs distinct state slots across the batch's rows", "state_slot")
-        if any(penalties_need_state(r) for r in self.specs):
+        if self._need_state:
             raise ValidationError("a row whose penalties count generated tokens must keep them in a state slot (ProcState) to take its "
                                   "step on the device: its CSR history would miss the drawn tokens", "state_slot")
 
@@ -361,23 +400,13 @@ class PackedBatch:
         qws_batch.advance); the rows' state slots must then be distinct."""
         if advance:
             self.check_advance()
-        b = Batch()
-        b.logits = logits.data_ptr()
-        b.dtype = DTYPE_BF16 if logits.dtype == torch.bfloat16 else DTYPE_F32
-        b.B, b.V = self.B, self.V
-        b.row_stride = logits.stride(0) if row_stride is None else row_stride
-        b.rows, b.hist, b.drafts = self.rows_t.data_ptr(), self.hist_t.data_ptr(), self.drafts_t.data_ptr()
-        b.bias_ids, b.bias_vals, b.stop_ids = self.bids_t.data_ptr(), self.bvals_t.data_ptr(), self.stops_t.data_ptr()
-        b.masks = self.masks_t.data_ptr() if self.masks_t is not None else None
-        b.mask_words = self.W
-        b.out_tokens = out_tokens.data_ptr()
-        b.out_logits = out_logits.data_ptr() if out_logits is not None else None
-        b.out_probs = out_probs.data_ptr() if out_probs is not None else None
-        b.out_info = out_info.data_ptr() if out_info is not None else None
-        if self.state is not None:
-            b.state_mem, b.state_slots = self.state.mem.data_ptr(), self.state.slots
-        b.advance = int(bool(advance))
-        return b
+        st = self.state
+        return Batch.from_buffer_copy(_BATCH.pack(
+            logits.data_ptr(), DTYPE_BF16 if logits.dtype == torch.bfloat16 else DTYPE_F32, self.B, self.V, logits.stride(0) if row_stride is None else row_stride,
+            self.rows_t.data_ptr(), self.hist_t.data_ptr(), self.drafts_t.data_ptr(), self.bids_t.data_ptr(), self.bvals_t.data_ptr(), self.stops_t.data_ptr(),
+            self.masks_t.data_ptr() if self.masks_t is not None else 0, self.W, out_tokens.data_ptr(), out_logits.data_ptr() if out_logits is not None else 0,
+            out_probs.data_ptr() if out_probs is not None else 0, out_info.data_ptr() if out_info is not None else 0,
+            st.mem.data_ptr() if st is not None else 0, st.slots if st is not None else 0, int(bool(advance))))
 
 
 class ProcState:
@@ -529,7 +558,7 @@ class Sampler:
             if t.device.type != "cuda" or not t.is_contiguous():
                 raise ValidationError("verify tensors must be contiguous CUDA tensors", "target_logits")
         if packed is None:
-            packed = PackedBatch(self.verify_rows(seqs, drafts.cpu().tolist()), V, target_logits.device, state)
+            packed = PackedBatch(self.verify_rows(seqs, drafts.cpu().tolist()), V, target_logits.device, state, ordered=True)
         if n_chain is not None and (n_chain.dtype != torch.int32 or n_chain.numel() != B or n_chain.device.type != "cuda"):
             raise ValidationError("n_chain must be a CUDA int32 [B] tensor", "n_chain")
         for name, t in (("out_probs", out_probs), ("out_logits", out_logits)):
@@ -569,7 +598,7 @@ class Sampler:
         B, Vd = draft_logits.shape
         if idmap.dtype != torch.int32 or idmap.numel() != Vd or idmap.device.type != "cuda" or not idmap.is_contiguous():
             raise ValidationError("idmap must be a contiguous CUDA int32 [Vd] tensor", "idmap")
-        packed = PackedBatch(rows, Vd, draft_logits.device)
+        packed = PackedBatch(rows, Vd, draft_logits.device, ordered=True)
         red = torch.empty(B, dtype=torch.int32, device=draft_logits.device)
         ids = torch.empty(B, dtype=torch.int32, device=draft_logits.device)
         q = torch.empty(B, Vd, dtype=torch.float32, device=draft_logits.device)  # every entry written by the call
@@ -580,18 +609,18 @@ class Sampler:
         return ids, q, red
 
     def sample(self, logits: torch.Tensor, rows: Sequence[RowSpec], state: Optional[ProcState] = None) -> torch.Tensor:
-        packed = PackedBatch(rows, logits.shape[1], logits.device, state)
+        packed = PackedBatch(rows, logits.shape[1], logits.device, state, ordered=True)
         return self.run(packed, logits)
 
     def processed_logits(self, logits: torch.Tensor, rows: Sequence[RowSpec], state: Optional[ProcState] = None) -> torch.Tensor:
-        packed = PackedBatch(rows, logits.shape[1], logits.device, state)
+        packed = PackedBatch(rows, logits.shape[1], logits.device, state, ordered=True)
         out = torch.empty(logits.shape, dtype=torch.float32, device=logits.device)
         self.run(packed, logits, out_logits=out)
         return out
 
     def probs(self, logits: torch.Tensor, rows: Sequence[RowSpec]):
         """(tokens, dense probabilities [B, V] (0 outside the kept set), info [B])."""
-        packed = PackedBatch(rows, logits.shape[1], logits.device)
+        packed = PackedBatch(rows, logits.shape[1], logits.device, ordered=True)
         probs = torch.zeros(logits.shape, dtype=torch.float32, device=logits.device)
         info = torch.empty(packed.B, dtype=torch.int32, device=logits.device)
         tok = self.run(packed, logits, out_probs=probs, out_info=info)

@@ -1,0 +1,63 @@
+"""The native id-list pass and the packed rows: the same arrays and refusals as the general Python path."""
+import numpy as np
+import pytest
+import torch
+
+import qwen_warp_amd as q
+from qwen_warp_amd import _lib
+from qwen_warp_amd.sampling import _ids
+
+V = 1000
+
+
+@pytest.mark.parametrize("n", [0, 1, 7, 5000])
+@pytest.mark.parametrize("kind", [list, tuple])
+def test_ids_native_pass(n, kind):
+    want = np.random.default_rng(n).integers(0, V, n)
+    got = _ids(kind(want.tolist()), V, "gen")
+    assert got.dtype == np.int64 and np.array_equal(got, want)
+    assert np.array_equal(_ids(kind(list(want)), V, "gen"), want)  # numpy integers: the general path
+
+
+@pytest.mark.parametrize("bad", [-1, V, 2 ** 31, 2 ** 70, True, 1.0, "1", None, np.bool_(True), np.float32(1)])
+def test_ids_refusals(bad):
+    for at in (0, 3):
+        ids = [1, 2, 3, 4]
+        ids[at] = bad
+        assert _lib.hostpack().ids(ids, V, np.empty(4, np.int64)) == -1
+        with pytest.raises(q.ValidationError):
+            _ids(ids, V, "gen")
+
+
+def test_ids_buffer_too_small():
+    assert _lib.hostpack().ids([1, 2, 3], V, np.empty(2, np.int64)) == -1
+
+
+def test_packed_rows_fields():
+    """The row words as the ctypes structure holds them, a value past its C field included (as the structure converts it)."""
+    rows = [q.RowSpec(temperature=0.7, top_k=2 ** 32 + 5, top_p=0.9, min_p=0.1, seed=-1, position=2 ** 33 + 1, row_key=-2, presence=1e39, gen=[1, 2], drafts=[3],
+                      bias={4: 0.5, 5: -1.0}, stop=[6, 7], min_tokens=9),
+            q.RowSpec(temperature=1.0, gen=[8, 9], repetition=1.5, allowed=[1, 33])]
+    p = q.PackedBatch(rows, V, "cpu")
+    a, b = p.host_rows[0], p.host_rows[1]
+    assert a.top_k == 5 and a.seed == 2 ** 64 - 1 and a.position == 1 and a.row_key == 2 ** 32 - 2 and a.presence == np.inf and a.proc_on == 1
+    assert (a.hist_off, a.n_prompt, a.n_gen, a.draft_off, a.n_drafts, a.bias_off, a.n_bias, a.stop_off, a.n_stop, a.ngen) == (0, 0, 2, 0, 1, 0, 2, 0, 2, 2)
+    assert (b.hist_off, b.n_gen, b.draft_off, b.mask_mode, b.mask_row, b.state_slot) == (2, 2, 1, _lib.MASK_ALLOWED, 0, -1)
+    assert bytes(p.host_rows) == p.rows_t.numpy().tobytes()
+    assert p.hist_t.tolist() == [1, 2, 8, 9] and p.bids_t.tolist() == [4, 5] and p.bvals_t.tolist() == [0.5, -1.0] and p.stops_t.tolist() == [6, 7]
+    assert p.masks_t[0].tolist()[:2] == [2, 2]
+    with pytest.raises(ValueError):
+        q.PackedBatch([q.RowSpec(banned=np.zeros(3, np.uint32))], V, "cpu")
+
+
+@pytest.mark.gpu
+def test_ordered_copies_back_to_back(sampler):
+    """Calls that pack their own rows, issued without waiting: each runs on its own rows (staging buffers are not reused early)."""
+    Vg = 8 * 4096
+    g = torch.Generator().manual_seed(1)
+    x = torch.randn(4, Vg, generator=g).cuda()
+    batches = [[q.RowSpec(temperature=1.0, top_p=0.9, repetition=1.3, gen=torch.randint(0, Vg, (2000,), generator=g).tolist(), seed=i, row_key=b) for b in range(4)]
+               for i in range(24)]
+    want = [sampler.run(q.PackedBatch(rows, Vg, "cuda"), x).tolist() for rows in batches]
+    got = [sampler.sample(x, rows) for rows in batches]
+    assert [t.tolist() for t in got] == want
