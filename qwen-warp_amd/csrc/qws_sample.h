@@ -208,7 +208,7 @@ struct RL {                      // k_resolve LDS views
   BI* bi;
   RS* st;
   float2* ts;
-  uint32_t* big;                 // [BLK]: a staged block
+  uint32_t* big;                 // [BIGW]: a staged block
   unsigned long long* fb;        // [MAXG][FB]: the staged power's bin words per block (first: the staged headers)
   unsigned long long* emu;       // [MAXG][NEXP]: the blocks' per-power mantissa sums
   uint64_t* ec;                  // [XG] gathered elements: comp
@@ -258,6 +258,28 @@ __device__ inline void block_range_u64(RS& st, unsigned long long mn, unsigned l
 // and the other lanes of its wave hit distinct LDS banks.
 constexpr int BIGW = BLK + BLK / 16;
 __device__ inline int big_at(int l) { return l + (l >> 4); }
+
+// k_resolve's LDS.  The rarer parts of a row (a min-p or top-k cut inside a bin, a top-p cut that the fast form does not
+// take, dense probabilities) are out-of-line functions that get it by one LDS pointer: inlined, with the selections'
+// several copies, the kernel was 76,000 instructions (ten times the instruction cache), and every launch fetches its
+// path anew.
+#define QWS_L __attribute__((address_space(3)))
+struct ResolveLds {
+  __attribute__((aligned(16))) unsigned long long fb[MAXG * FB];
+  unsigned long long emu[MAXG * NEXP];
+  uint64_t ec[XG];
+  uint32_t em[XG];
+  __attribute__((aligned(16))) uint32_t big[BIGW];
+  __attribute__((aligned(16))) float2 ts[1024];
+  __attribute__((aligned(16))) u128 red[NWV2 + 1];
+  RS st;
+  BI bi[MAXG];
+  qws_batch B;                   // the call's arguments and the row, for the out-of-line parts
+  qws_row R;
+  int nt;
+};
+__device__ __forceinline__ RL rl_of(ResolveLds& S) { return RL{S.bi, &S.st, S.ts, S.big, S.fb, S.emu, S.ec, S.em, &S.nt, S.red}; }
+__device__ __forceinline__ char* uniform_ptr(char* p) { return (char*)readlane<uint64_t>((uint64_t)p, 0); }
 
 // A block's raw values as the stager loads them: the logits (thread layout of Blk), the mask words and the patches.
 template <int DT>
@@ -329,8 +351,9 @@ __device__ __forceinline__ void stage_block_body(const RL& L, const qws_batch& B
 // The out-of-line copy for the rare rescans (the draw stages its block inline: a call would spill the caller's
 // registers to scratch around it).
 template <int DT>
-__device__ __noinline__ void stage_block(const RL& L, const qws_batch& B, const qws_row& R, char* ws, int row, int g) {
-  stage_block_body<DT>(L, B, R, ws, row, g);
+__device__ __noinline__ void stage_block(QWS_L ResolveLds* s, char* ws, int row, int g) {
+  ResolveLds& S = *(ResolveLds*)s;
+  stage_block_body<DT>(rl_of(S), S.B, S.R, uniform_ptr(ws), __builtin_amdgcn_readfirstlane(row), __builtin_amdgcn_readfirstlane(g));
 }
 
 // The fine bins of row power p of every block into L.fb and summed over the row into st.fcnt / st.fmu.  Bins a block
@@ -493,8 +516,9 @@ __device__ inline XRange bin_xrange(int qb, float K) {
 // Calls fn(comp, mu) for every candidate of row bin rb (gathered: from LDS; else from the blocks' lists and rescans).
 // All threads; ends with a barrier.
 template <int DT, typename F>
-__device__ __forceinline__ void for_bin(const RL& L, const qws_batch& B, const qws_row& R, char* ws, int row, F fn) {
+__device__ __forceinline__ void for_bin(ResolveLds& S, char* ws, int row, F fn) {
   using BL = Blk<DT, NT2>;
+  const RL L = rl_of(S);
   const RS& st = *L.st;
   const int tid = threadIdx.x;
   if (st.gstaged) {
@@ -511,7 +535,7 @@ __device__ __forceinline__ void for_bin(const RL& L, const qws_batch& B, const q
   }
   for (int g = 0; g < (st.gres ? G : 0); g++) {
     if (L.bi[g].gsrc != 2) continue;
-    stage_block<DT>(L, B, R, ws, row, g);
+    stage_block<DT>((QWS_L ResolveLds*)&S, ws, row, g);
     const float* xs = (const float*)L.big;
     const int t0 = tid * BL::EPT;
 #pragma unroll
@@ -525,11 +549,126 @@ __device__ __forceinline__ void for_bin(const RL& L, const qws_batch& B, const q
   bar();
 }
 
+// The blocks of st.gfast rescanned for the elements of row bin rb, into the gathered list.  Out of line: the rare path's
+// registers would spill the resolver's other paths.  All threads.
+template <int DT>
+__device__ __noinline__ void rescan_fast(QWS_L ResolveLds* s, char* ws_, int row_, int rb_) {
+  using BL = Blk<DT, NT2>;
+  ResolveLds& S = *(ResolveLds*)s;
+  const RL L = rl_of(S);
+  const qws_batch& B = S.B;
+  const qws_row& R = S.R;
+  RS& st = *L.st;
+  char* const ws = uniform_ptr(ws_);
+  const int row = __builtin_amdgcn_readfirstlane(row_), rb = __builtin_amdgcn_readfirstlane(rb_);
+  const int G = __builtin_amdgcn_readfirstlane(st.G), tid = threadIdx.x;
+  unsigned long long mn = ~0ull, mx = 0ull;
+  // blocks whose processed tokens are all recorded as patches: raw logits straight into registers, RB blocks at once
+  // (all their loads in flight together); only the bin's elements are weighed, each placed at its block's next
+  // slot.  Masked and processed tokens are marked in a bitmap per block (in L.big) that the raw values found are
+  // tested against, and the patches' values are tested themselves.  (Through the staged block, one at a time, a
+  // block costs ~5 us: rows that missed 20-30 blocks took 75-150 us in all.)
+  constexpr int RB = 8;  // the resolver runs one workgroup per CU: registers for eight blocks of loads in flight
+  constexpr int BW32 = BLK / 32;
+  static_assert(RB * BW32 <= BIGW && NT2 == 2 * BW32 && TCAP == 2 * NT2, "bitmap words and patches per thread");
+  uint32_t* const bm = L.big;
+  const uint32_t flip = R.mask_mode == QWS_MASK_ALLOWED ? 0xFFFFFFFFu : 0u;
+  const unsigned* const mrow = B.masks + (R.mask_mode ? (size_t)R.mask_row * (size_t)B.mask_words : 0);
+  const int qb = st.row_top - rb;  // the bin's floor(t) >> 4
+  const float K = st.K;
+  const XRange xr = bin_xrange(qb, K);
+  auto place = [&](BI& b, int g, int local, float v) {  // the value v of block g's token, when it lies in the bin
+    const float t = tval(v, K);
+    if (v == v && v != -INFINITY && (tfloor(t) >> 4) == qb) {  // NaN counts as -inf
+      const int p = b.gofs + atomicAdd(&b.goff, 1);
+      const uint64_t c = comp(okey(v), (uint32_t)(g * BLK + local));
+      mn = c < mn ? c : mn;
+      mx = c > mx ? c : mx;
+      if (p < XG) {  // always: the bin words count these elements
+        L.ec[p] = c;
+        L.em[p] = weigh(t, L.ts).mu;
+      }
+    }
+  };
+  unsigned long long fm = readlane<unsigned long long>(st.gfast, 0);  // in scalar registers: the batches branch on it
+  while (fm) {
+    int gb[RB];
+#pragma unroll
+    for (int k = 0; k < RB; k++) {
+      gb[k] = fm ? __ffsll((long long)fm) - 1 : -1;
+      fm &= fm - 1ull;
+    }
+    // every load issued before any is used; an unused slot loads nothing (one CU reads a block at ~16 bytes per cycle)
+    float x[RB][BL::EPT];
+#pragma unroll
+    for (int k = 0; k < RB; k++) {
+      if (gb[k] >= 0) BL::load_raw(B, row, gb[k] * BLK, min(B.V, gb[k] * BLK + BLK), x[k]);  // uniform; -inf past V
+    }
+    bool marks = R.mask_mode != 0;  // uniform
+#pragma unroll
+    for (int k = 0; k < RB; k++) marks = marks || (gb[k] >= 0 && L.bi[gb[k]].n_patch > 0);
+    if (marks) {
+      const int hw = tid / BW32, wi = tid % BW32;
+      uint32_t mv[RB / 2];
+#pragma unroll
+      for (int k = 0; k < RB / 2; k++) {
+        const int gk = hw ? gb[2 * k + 1] : gb[2 * k], i = gk * BW32 + wi;
+        mv[k] = R.mask_mode && gk >= 0 && i * 32 < B.V ? gmem(mrow)[i] ^ flip : 0u;
+      }
+      bar();  // the bitmaps of the batch before are read no more
+#pragma unroll
+      for (int k = 0; k < RB / 2; k++) bm[(2 * k + hw) * BW32 + wi] = mv[k];
+      bar();
+      for (int i = tid; i < TCAP; i += NT2) {  // two rounds of patches at most, the blocks' loads of a round together
+        unsigned long long pv[RB];
+        bool more = false;
+#pragma unroll
+        for (int k = 0; k < RB; k++) {
+          const int np = gb[k] >= 0 ? L.bi[gb[k]].n_patch : 0;
+          more = more || np > NT2;
+          pv[k] = i < np ? gmem((const unsigned long long*)(rec_of(ws, G, row, max(gb[k], 0)) + PATCH_OFF))[i] : 0xFFFFFFFFull;  // local ~0: none
+        }
+#pragma unroll
+        for (int k = 0; k < RB; k++) {
+          const uint32_t l = (uint32_t)pv[k];
+          if (l != 0xFFFFFFFFu) {
+            atomicOr(&bm[k * BW32 + (l >> 5)], 1u << (l & 31));
+            const float v = __uint_as_float((uint32_t)(pv[k] >> 32));
+            if (xr.maybe(v)) place(L.bi[gb[k]], gb[k], (int)l, v);
+          }
+        }
+        if (!more) break;  // uniform
+      }
+      bar();
+    }
+#pragma unroll
+    for (int k = 0; k < RB; k++) {
+      if (gb[k] < 0) continue;
+      BI& b = L.bi[gb[k]];
+#pragma unroll
+      for (int e = 0; e < BL::EPT; e++) {
+        const float v = x[k][e];
+        if (!xr.maybe(v)) continue;  // NaN fails it too
+        const int l = BL::local(e);
+        if (marks && ((bm[k * BW32 + (l >> 5)] >> (l & 31)) & 1u)) continue;
+        place(b, gb[k], l, v);
+      }
+    }
+  }
+  mn = wave_min_u64(mn);
+  mx = wave_max_u64(mx);
+  if (lane_id() == 0) {
+    atomicMin(&st.gmin, mn);
+    atomicMax(&st.gmax, mx);
+  }
+}
+
 // Gathers row bin rb (its power's fine bins staged): each block's elements come from its list when its window held
-// the bin, else from a rescan of the block.  The bin is held in LDS when it has at most XG elements.  SKIP: a batch of
-// rescans loads only its blocks (the verify rows' instance).  All threads.
-template <int DT, bool SKIP>
-__device__ __forceinline__ void gather(const RL& L, const qws_batch& B, const qws_row& R, char* ws, int row, int rb) {
+// the bin, else from a rescan of the block.  The bin is held in LDS when it has at most XG elements.  All threads.
+template <int DT>
+__device__ __forceinline__ void gather(ResolveLds& S, char* ws, int row, int rb) {
+  const RL L = rl_of(S);
+  const qws_row& R = S.R;
   RS& st = *L.st;
   const int G = st.G, tid = threadIdx.x;
   if (st.gbin == rb) return;  // uniform: st.gbin is written only after the barrier below, which every wave passes after this test
@@ -606,111 +745,11 @@ __device__ __forceinline__ void gather(const RL& L, const qws_batch& B, const qw
     }
     bar();
     using BL = Blk<DT, NT2>;
-    {
-      // blocks whose processed tokens are all recorded as patches: raw logits straight into registers, RB blocks at once
-      // (all their loads in flight together); only the bin's elements are weighed, each placed at its block's next
-      // slot.  Masked and processed tokens are marked in a bitmap per block (in L.big) that the raw values found are
-      // tested against, and the patches' values are tested themselves.  (Through the staged block, one at a time, a
-      // block costs ~5 us: rows that missed 20-30 blocks took 75-150 us in all.)
-      constexpr int RB = 8;  // the resolver runs one workgroup per CU: registers for eight blocks of loads in flight
-      constexpr int BW32 = BLK / 32;
-      static_assert(RB * BW32 <= BIGW && NT2 == 2 * BW32 && TCAP == 2 * NT2, "bitmap words and patches per thread");
-      uint32_t* const bm = L.big;
-      const uint32_t flip = R.mask_mode == QWS_MASK_ALLOWED ? 0xFFFFFFFFu : 0u;
-      const unsigned* const mrow = B.masks + (R.mask_mode ? (size_t)R.mask_row * (size_t)B.mask_words : 0);
-      const int qb = st.row_top - rb;  // the bin's floor(t) >> 4
-      const float K = st.K;
-      const XRange xr = bin_xrange(qb, K);
-      auto place = [&](BI& b, int g, int local, float v) {  // the value v of block g's token, when it lies in the bin
-        const float t = tval(v, K);
-        if (v == v && v != -INFINITY && (tfloor(t) >> 4) == qb) {  // NaN counts as -inf
-          const int p = b.gofs + atomicAdd(&b.goff, 1);
-          const uint64_t c = comp(okey(v), (uint32_t)(g * BLK + local));
-          mn = c < mn ? c : mn;
-          mx = c > mx ? c : mx;
-          if (p < XG) {  // always: the bin words count these elements
-            L.ec[p] = c;
-            L.em[p] = weigh(t, L.ts).mu;
-          }
-        }
-      };
-      unsigned long long fm = st.gfast;  // uniform
-      while (fm) {
-        int gb[RB];
-#pragma unroll
-        for (int k = 0; k < RB; k++) {
-          gb[k] = fm ? __ffsll((long long)fm) - 1 : -1;
-          fm &= fm - 1ull;
-        }
-        // every load issued before any is used.  SKIP (the verify rows' instance): an unused slot loads nothing, since
-        // one CU reads a block at ~16 bytes per cycle; the sampling rows' instance reads the first block again there
-        // instead (no branch around the loads: the skipping code slowed that kernel's other paths by its layout)
-        float x[RB][BL::EPT];
-#pragma unroll
-        for (int k = 0; k < RB; k++) {
-          if constexpr (SKIP) {
-            if (gb[k] >= 0) BL::load_raw(B, row, gb[k] * BLK, min(B.V, gb[k] * BLK + BLK), x[k]);  // uniform; -inf past V
-          } else {
-            const int gk = gb[k] >= 0 ? gb[k] : gb[0];
-            BL::load_raw(B, row, gk * BLK, min(B.V, gk * BLK + BLK), x[k]);  // -inf past V; NaN tested below
-          }
-        }
-        bool marks = R.mask_mode != 0;  // uniform
-#pragma unroll
-        for (int k = 0; k < RB; k++) marks = marks || (gb[k] >= 0 && L.bi[gb[k]].n_patch > 0);
-        if (marks) {
-          uint2 pv[RB][2];
-#pragma unroll
-          for (int k = 0; k < RB; k++) {
-            const int np = gb[k] >= 0 ? L.bi[gb[k]].n_patch : 0;
-            const QWS_G unsigned long long* PT = gmem((const unsigned long long*)(rec_of(ws, G, row, max(gb[k], 0)) + PATCH_OFF));
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-              const unsigned long long w = tid + i * NT2 < np ? PT[tid + i * NT2] : 0xFFFFFFFFull;  // local ~0: none
-              pv[k][i] = make_uint2((uint32_t)w, (uint32_t)(w >> 32));
-            }
-          }
-          const int hw = tid / BW32, wi = tid % BW32;
-          uint32_t mv[RB / 2];
-#pragma unroll
-          for (int k = 0; k < RB / 2; k++) {
-            const int gk = hw ? gb[2 * k + 1] : gb[2 * k], i = gk * BW32 + wi;
-            mv[k] = R.mask_mode && gk >= 0 && i * 32 < B.V ? gmem(mrow)[i] ^ flip : 0u;
-          }
-          bar();  // the bitmaps of the batch before are read no more
-#pragma unroll
-          for (int k = 0; k < RB / 2; k++) bm[(2 * k + hw) * BW32 + wi] = mv[k];
-          bar();
-#pragma unroll
-          for (int k = 0; k < RB; k++)
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-              if (pv[k][i].x != 0xFFFFFFFFu) {
-                atomicOr(&bm[k * BW32 + (pv[k][i].x >> 5)], 1u << (pv[k][i].x & 31));
-                const float v = __uint_as_float(pv[k][i].y);
-                if (xr.maybe(v)) place(L.bi[gb[k]], gb[k], (int)pv[k][i].x, v);
-              }
-          bar();
-        }
-#pragma unroll
-        for (int k = 0; k < RB; k++) {
-          if (gb[k] < 0) continue;
-          BI& b = L.bi[gb[k]];
-#pragma unroll
-          for (int e = 0; e < BL::EPT; e++) {
-            const float v = x[k][e];
-            if (!xr.maybe(v)) continue;  // NaN fails it too
-            const int l = BL::local(e);
-            if (marks && ((bm[k * BW32 + (l >> 5)] >> (l & 31)) & 1u)) continue;
-            place(b, gb[k], l, v);
-          }
-        }
-      }
-    }
+    if (st.gfast) rescan_fast<DT>((QWS_L ResolveLds*)&S, ws, row, rb);  // uniform
     for (unsigned long long sm = st.gslow; sm; sm &= sm - 1ull) {  // uniform: read after the barrier
       const int g = __ffsll((long long)sm) - 1;
       if (tid == 0) L.bi[g].gofs = st.si[7];  // the block's elements follow (their order within the block is free)
-      stage_block<DT>(L, B, R, ws, row, g);
+      stage_block<DT>((QWS_L ResolveLds*)&S, ws, row, g);
       const float* xs = (const float*)L.big;
       const int t0 = tid * BL::EPT;
 #pragma unroll
@@ -750,9 +789,9 @@ __device__ __forceinline__ void gather(const RL& L, const qws_batch& B, const qw
 // select_rounds: the rounds from the comp range [kmin, kmax] with value base before it.  All threads, after a barrier
 // that follows the last reads of the buckets.
 template <int DT>
-__device__ __forceinline__ void select_rounds(const RL& L, const qws_batch& B, const qws_row& R, char* ws, int row, bool by_mass, uint64_t target,
+__device__ __forceinline__ void select_rounds(ResolveLds& S, char* ws, int row, bool by_mass, uint64_t target,
                                               uint64_t kmin, uint64_t kmax, uint64_t base) {
-  RS& st = *L.st;
+  RS& st = S.st;
   const int tid = threadIdx.x;
   for (int round = 0; round < 16; round++) {
     const int sh = bucket_shift(kmax - kmin);
@@ -761,7 +800,7 @@ __device__ __forceinline__ void select_rounds(const RL& L, const qws_batch& B, c
       st.bsum[i] = 0;
     }
     bar();
-    for_bin<DT>(L, B, R, ws, row, [&](uint64_t c, uint32_t mu) {
+    for_bin<DT>(S, ws, row, [&](uint64_t c, uint32_t mu) {
       if (c >= kmin && c <= kmax) {
         const int b = NBK - 1 - (int)((c - kmin) >> sh);  // bucket 0 = the largest comps
         atomicAdd(&st.bcnt[b], 1u);
@@ -805,7 +844,7 @@ __device__ __forceinline__ void select_rounds(const RL& L, const qws_batch& B, c
     if (nb <= 64) {  // at most a wave of elements left: wave 0 ranks them directly
       if (tid == 0) st.si[3] = 0;
       bar();
-      for_bin<DT>(L, B, R, ws, row, [&](uint64_t c, uint32_t mu) {
+      for_bin<DT>(S, ws, row, [&](uint64_t c, uint32_t mu) {
         if (c >= bl && c <= bh) {
           const int p = atomicAdd(&st.si[3], 1);
           if (p < 64) {  // always: the bucket held nb <= 64 of them
@@ -839,11 +878,11 @@ __device__ __forceinline__ void select_rounds(const RL& L, const qws_batch& B, c
 }
 // select_in_bin: the selection over the gathered bin (gather called first).  All threads.
 template <int DT>
-__device__ __forceinline__ void select_in_bin(const RL& L, const qws_batch& B, const qws_row& R, char* ws, int row, bool by_mass, uint64_t target) {
-  RS& st = *L.st;
+__device__ __forceinline__ void select_in_bin(ResolveLds& S, char* ws, int row, bool by_mass, uint64_t target) {
+  RS& st = S.st;
   if (!st.gstaged) {
     unsigned long long mn = ~0ull, mx = 0ull;
-    for_bin<DT>(L, B, R, ws, row, [&](uint64_t c, uint32_t) {
+    for_bin<DT>(S, ws, row, [&](uint64_t c, uint32_t) {
       mn = c < mn ? c : mn;
       mx = c > mx ? c : mx;
     });
@@ -853,7 +892,7 @@ __device__ __forceinline__ void select_in_bin(const RL& L, const qws_batch& B, c
   }
   const uint64_t kmin = st.gstaged ? st.gmin : st.kmin, kmax = st.gstaged ? st.gmax : st.kmax;
   if (kmin > kmax) return;
-  select_rounds<DT>(L, B, R, ws, row, by_mass, target, kmin, kmax, 0ull);
+  select_rounds<DT>(S, ws, row, by_mass, target, kmin, kmax, 0ull);
 }
 
 // The gather and selection of row bin rb together, for a bin whose elements all lie in their blocks' lists and fit
@@ -868,8 +907,10 @@ __device__ __forceinline__ void select_in_bin(const RL& L, const qws_batch& B, c
 constexpr int XS = XG / NT2;  // elements per thread
 static_assert(XG % NT2 == 0 && MAXG <= 64, "select_listed layout");
 template <int DT>
-__device__ __forceinline__ bool select_listed(const RL& L, const qws_batch& B, const qws_row& R, char* ws, int row, int rb, bool by_mass, uint64_t target,
+__device__ __forceinline__ bool select_listed(ResolveLds& S, char* ws, int row, int rb, bool by_mass, uint64_t target,
                                               uint64_t* cut, uint64_t* incl) {
+  const RL L = rl_of(S);
+  const qws_row& R = S.R;
   RS& st = *L.st;
   const int G = st.G, tid = threadIdx.x, lane = lane_id();
   if (st.gbin == rb || (R.test_flags & (QWS_TF_RESCAN | QWS_TF_SPLIT_SELECT))) return false;  // uniform: st.gbin is written after the first barrier below
@@ -995,7 +1036,7 @@ __device__ __forceinline__ bool select_listed(const RL& L, const qws_batch& B, c
   const uint64_t bh = kmax - bl <= span ? kmax : bl + span;
   if (nb > 64) {  // more rounds, over the elements in LDS
     bar();
-    select_rounds<DT>(L, B, R, ws, row, by_mass, target, bl, bh, base);
+    select_rounds<DT>(S, ws, row, by_mass, target, bl, bh, base);
     *cut = st.su[4];
     *incl = st.su[5];
     return true;
@@ -1330,6 +1371,7 @@ struct TopRow {
   uint32_t u_draw;
   float temperature, top_p, min_p;
   double log2_min_p;
+  unsigned long long thr_lo, thr_hi;       // finish_small: the top-p threshold (row units), 0 = from top_p over the candidates
   int* out_tokens;
   int* out_info;
   float* out_probs;
@@ -1355,6 +1397,104 @@ __device__ inline u128 wave_scan_weights(uint64_t v) {
   const int row = lane_id() >> 4;
   const u128 b1 = r0, b2 = b1 + r1, b3 = b2 + r2;
   return (u128)v + (row == 0 ? (u128)0 : row == 1 ? b1 : row == 2 ? b2 : b3);
+}
+// The row's token from n <= TOP_NL1 distinct candidates (src, zeros past them to TOP_NL1), among which are its best
+// min(top_k, 64) and, with a threshold given, every one down to its crossing: ranked by counting, then one per lane in
+// rank order weighed, cut by top-k, min-p and top-p, and drawn from in index order.  All threads; ends with a barrier.
+template <bool VER>
+__device__ __forceinline__ int finish_ranked(const TopRow& A, int n, const uint64_t* src, const float2* ts, TopBuf& L) {
+  const int tid = threadIdx.x, lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(wave_id());
+  const int K = A.K;
+  {  // ranks by counting: thread (i, p) counts the larger ones of entries [32 p, 32 p + 32)
+    const int i = tid & (TOP_NL1 - 1), p = tid / TOP_NL1;
+    const uint64_t ci = src[i];
+    uint32_t r = 0;
+    if (TOP_NL1 / 4 * p < n) {  // uniform in the wave
+#pragma unroll
+      for (int j = 0; j < TOP_NL1 / 4; j++) r += src[TOP_NL1 / 4 * p + j] > ci ? 1u : 0u;
+    }
+    L.rk[p][i] = r;
+    bar();
+    if (tid < n) {  // n <= TOP_NL1: p = 0
+      const uint32_t rank = L.rk[0][tid] + L.rk[1][tid] + L.rk[2][tid] + L.rk[3][tid];
+      if (rank < (uint32_t)K) L.srt[rank] = ci;
+    }
+    bar();
+  }
+  // every wave: the row's candidates (top-k applied), one per lane in rank order, weighed and cut by min-p and top-p
+  const int m0 = min(n, K);
+  const uint64_t cc = lane < m0 ? L.srt[lane] : 0ull;
+  const uint32_t idx = comp_idx(cc);
+  const float Ks = kscale(A.temperature);
+  const float t = tval(okey_val(comp_key(cc)), Ks);
+  const float tmax = readlane<float>(t, 0);
+  const int row_top = (tfloor(tmax) >> 10) * FB + (FB - 1);
+  const W ww = weigh(lane < m0 ? t : 0.0f, ts);
+  const int r = row_top - (tfloor(t) >> 4);
+  bool keep = lane < m0 && r < NR;
+  if (A.min_p > 0.0f) keep = keep && t >= (float)((double)(tmax / 1024.0f) + A.log2_min_p) * 1024.0f;
+  uint64_t w = keep ? rw1(ww.mu, r) : 0ull;
+  const u128 incl = wave_scan_weights(w);
+  u128 S2 = readlane<u128>(incl, 63);
+  int m = __popcll(__ballot(w != 0));  // weighted candidates: lanes 0 .. m - 1
+  {
+    u128 thr = ld128(A.thr_lo, A.thr_hi);
+    if (thr == 0 && A.top_p < 1.0f) thr = mul_shr_ceil(S2, (uint64_t)floor((double)A.top_p * 4294967296.0), 32);
+    if (thr > 0) {
+      m = min(first_lane(w != 0 && thr <= incl), 63) + 1;  // thr <= S2: one lane crosses
+      S2 = readlane<u128>(incl, m - 1);
+      w = lane < m ? w : 0ull;
+    }
+  }
+  // the draw in index order: wave p sums, for each candidate, the kept weights of candidates [8 p, 8 p + 8) with a lower
+  // index (below 2^62), wave 0 adds the eight sums up
+  if (wave * 8 < m) {  // uniform in the wave
+    uint64_t b = 0;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const uint32_t ij = readlane<uint32_t>(idx, wave * 8 + j);
+      const uint64_t wj = readlane<uint64_t>(w, wave * 8 + j);
+      b += ij < idx ? wj : 0ull;
+    }
+    L.part[wave][lane] = b;
+  }
+  bar();
+  if (wave == 0) {
+    const u128 tt = mul_shr_floor(S2, A.u_draw, 24);
+    u128 below = 0;
+#pragma unroll
+    for (int p = 0; p < NWV2; p++)
+      if (p * 8 < m) below += L.part[p][lane];
+    const int l = first_lane(w != 0 && below <= tt && tt < below + w);
+    const int tok = l < 64 ? (int)readlane<uint32_t>(idx, l) : (n == 0 ? 0 : -1);  // no candidate: token 0, as a greedy row's
+    if (A.out_probs && lane < m) {  // k_scan has written zeros
+      const double S2d = (double)(uint64_t)(S2 >> 64) * 18446744073709551616.0 + (double)(uint64_t)S2;
+      A.out_probs[(size_t)A.row * A.V + idx] = (float)((double)w / S2d);
+    }
+    const int rl = readlane<int>(r, max(m - 1, 0));
+    const uint64_t cl = readlane<uint64_t>(cc, max(m - 1, 0));
+    if (lane == 0) {
+      A.out_tokens[A.row] = tok;
+      if (A.out_info) A.out_info[A.row] = n == 0 ? 2 : tok < 0 ? -1 : 0;
+      if (VER) {
+        RowRes o = {};
+        o.kind = n == 0 ? RR_EMPTY : tok < 0 ? RR_FAIL : RR_SAMPLED;
+        o.tok = tok;
+        if (n != 0) {
+          o.s_lo = (unsigned long long)S2;
+          o.s_hi = (unsigned long long)(S2 >> 64);
+          o.cC = cl;  // the kept set: the rank prefix down to its last member
+          o.cR = rl;
+          o.row_top = row_top;
+          o.K = Ks;
+        }
+        A.rres[A.row] = o;
+      }
+      L.tok = tok;
+    }
+  }
+  bar();
+  return __builtin_amdgcn_readfirstlane(L.tok);
 }
 template <bool VER>
 __device__ __forceinline__ int resolve_top_body(const TopRow& A, const char* hdrs, const float2* ts, TopBuf& L) {
@@ -1416,100 +1556,10 @@ __device__ __forceinline__ int resolve_top_body(const TopRow& A, const char* hdr
     n = __builtin_amdgcn_readfirstlane(L.cnt);
     src = L.mxs;
   }
-  {  // ranks by counting: thread (i, p) counts the larger ones of entries [32 p, 32 p + 32)
-    const int i = tid & (TOP_NL1 - 1), p = tid / TOP_NL1;
-    const uint64_t ci = src[i];
-    uint32_t r = 0;
-    if (TOP_NL1 / 4 * p < n) {  // uniform in the wave
-#pragma unroll
-      for (int j = 0; j < TOP_NL1 / 4; j++) r += src[TOP_NL1 / 4 * p + j] > ci ? 1u : 0u;
-    }
-    L.rk[p][i] = r;
-    bar();
-    if (tid < n) {  // n <= TOP_NL1: p = 0
-      const uint32_t rank = L.rk[0][tid] + L.rk[1][tid] + L.rk[2][tid] + L.rk[3][tid];
-      if (rank < (uint32_t)K) L.srt[rank] = ci;
-    }
-    bar();
-  }
-  // every wave: the row's candidates (top-k applied), one per lane in rank order, weighed and cut by min-p and top-p
-  const int m0 = min(n, K);
-  const uint64_t cc = lane < m0 ? L.srt[lane] : 0ull;
-  const uint32_t idx = comp_idx(cc);
-  const float Ks = kscale(A.temperature);
-  const float t = tval(okey_val(comp_key(cc)), Ks);
-  const float tmax = readlane<float>(t, 0);
-  const int row_top = (tfloor(tmax) >> 10) * FB + (FB - 1);
-  const W ww = weigh(lane < m0 ? t : 0.0f, ts);
-  const int r = row_top - (tfloor(t) >> 4);
-  bool keep = lane < m0 && r < NR;
-  if (A.min_p > 0.0f) keep = keep && t >= (float)((double)(tmax / 1024.0f) + A.log2_min_p) * 1024.0f;
-  uint64_t w = keep ? rw1(ww.mu, r) : 0ull;
-  const u128 incl = wave_scan_weights(w);
-  u128 S2 = readlane<u128>(incl, 63);
-  int m = __popcll(__ballot(w != 0));  // weighted candidates: lanes 0 .. m - 1
-  if (A.top_p < 1.0f) {
-    const u128 thr = mul_shr_ceil(S2, (uint64_t)floor((double)A.top_p * 4294967296.0), 32);
-    if (thr > 0) {
-      m = min(first_lane(w != 0 && thr <= incl), 63) + 1;  // thr <= S2: one lane crosses
-      S2 = readlane<u128>(incl, m - 1);
-      w = lane < m ? w : 0ull;
-    }
-  }
-  // the draw in index order: wave p sums, for each candidate, the kept weights of candidates [8 p, 8 p + 8) with a lower
-  // index (below 2^62), wave 0 adds the eight sums up
-  if (wave * 8 < m) {  // uniform in the wave
-    uint64_t b = 0;
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const uint32_t ij = readlane<uint32_t>(idx, wave * 8 + j);
-      const uint64_t wj = readlane<uint64_t>(w, wave * 8 + j);
-      b += ij < idx ? wj : 0ull;
-    }
-    L.part[wave][lane] = b;
-  }
-  bar();
-  if (wave == 0) {
-    const u128 tt = mul_shr_floor(S2, A.u_draw, 24);
-    u128 below = 0;
-#pragma unroll
-    for (int p = 0; p < NWV2; p++)
-      if (p * 8 < m) below += L.part[p][lane];
-    const int l = first_lane(w != 0 && below <= tt && tt < below + w);
-    const int tok = l < 64 ? (int)readlane<uint32_t>(idx, l) : (n == 0 ? 0 : -1);  // no candidate: token 0, as a greedy row's
-    if (A.out_probs && lane < m) {  // k_scan has written zeros
-      const double S2d = (double)(uint64_t)(S2 >> 64) * 18446744073709551616.0 + (double)(uint64_t)S2;
-      A.out_probs[(size_t)A.row * A.V + idx] = (float)((double)w / S2d);
-    }
-    const int rl = readlane<int>(r, max(m - 1, 0));
-    const uint64_t cl = readlane<uint64_t>(cc, max(m - 1, 0));
-    if (lane == 0) {
-      A.out_tokens[A.row] = tok;
-      if (A.out_info) A.out_info[A.row] = n == 0 ? 2 : tok < 0 ? -1 : 0;
-      if (VER) {
-        RowRes o = {};
-        o.kind = n == 0 ? RR_EMPTY : tok < 0 ? RR_FAIL : RR_SAMPLED;
-        o.tok = tok;
-        if (n != 0) {
-          o.s_lo = (unsigned long long)S2;
-          o.s_hi = (unsigned long long)(S2 >> 64);
-          o.cC = cl;  // the kept set: the rank prefix down to its last member
-          o.cR = rl;
-          o.row_top = row_top;
-          o.K = Ks;
-        }
-        A.rres[A.row] = o;
-      }
-      L.tok = tok;
-    }
-  }
-  bar();
-  return __builtin_amdgcn_readfirstlane(L.tok);
+  return finish_ranked<VER>(A, n, src, ts, L);
 }
-#define QWS_L __attribute__((address_space(3)))
-// The call passes the row's arguments through LDS (an out-of-line function's arguments would arrive in vector registers)
-template <bool VER>
-__device__ __noinline__ int resolve_top(QWS_L const TopRow* a, QWS_L const char* hdrs, QWS_L const float2* ts, QWS_L char* buf) {
+// The calls pass the row's arguments through LDS (an out-of-line function's arguments would arrive in vector registers)
+__device__ __forceinline__ TopRow top_row(QWS_L const TopRow* a) {
   TopRow A;
   A.row = __builtin_amdgcn_readfirstlane(a->row);
   A.V = __builtin_amdgcn_readfirstlane(a->V);
@@ -1520,40 +1570,142 @@ __device__ __noinline__ int resolve_top(QWS_L const TopRow* a, QWS_L const char*
   A.top_p = a->top_p;
   A.min_p = a->min_p;
   A.log2_min_p = a->log2_min_p;
+  A.thr_lo = a->thr_lo;
+  A.thr_hi = a->thr_hi;
   A.out_tokens = a->out_tokens;
   A.out_info = a->out_info;
   A.out_probs = a->out_probs;
   A.rres = a->rres;
-  return resolve_top_body<VER>(A, (const char*)hdrs, (const float2*)ts, *(TopBuf*)(char*)buf);
+  return A;
+}
+template <bool VER>
+__device__ __noinline__ int resolve_top(QWS_L const TopRow* a, QWS_L const char* hdrs, QWS_L const float2* ts, QWS_L char* buf) {
+  return resolve_top_body<VER>(top_row(a), (const char*)hdrs, (const float2*)ts, *(TopBuf*)(char*)buf);
+}
+// finish_ranked over the n candidates in the buffer's list
+template <bool VER>
+__device__ __noinline__ int finish_small(QWS_L const TopRow* a, int n, QWS_L const float2* ts, QWS_L char* buf) {
+  TopBuf& L = *(TopBuf*)(char*)buf;
+  return finish_ranked<VER>(top_row(a), __builtin_amdgcn_readfirstlane(n), L.lst, (const float2*)ts, L);
+}
+
+// ---------------------------------------------------------------------------------------------- out-of-line parts of a row
+// (each uniform arguments, all threads; results in the row state after a barrier)
+// The min-p cut inside row bin rc (its power staged): the cut's comp -> st.su[4], the bin's kept candidates -> st.su[5]
+template <int DT>
+__device__ __noinline__ void minp_cut(QWS_L ResolveLds* s, char* ws_, int row_, int rc_, float tcut) {
+  ResolveLds& S = *(ResolveLds*)s;
+  char* const ws = uniform_ptr(ws_);
+  const int row = __builtin_amdgcn_readfirstlane(row_), rc = __builtin_amdgcn_readfirstlane(rc_);
+  RS& st = S.st;
+  const float K = st.K;
+  gather<DT>(S, ws, row, rc);
+  unsigned long long v = 0;  // kept: t >= tcut, a prefix of the bin in comp order
+  for_bin<DT>(S, ws, row, [&](uint64_t c, uint32_t) { v += tval(okey_val(comp_key(c)), K) >= tcut ? 1ull : 0ull; });
+  block_add_u64(st, v);
+  const unsigned long long nk = st.su[7];
+  uint64_t cC;
+  float xc;
+  if (nk == 0) {
+    cC = ~0ull;
+  } else if (nk == (unsigned long long)st.gn) {
+    cC = 0;
+  } else if (first_x_t(tcut, K, &xc)) {  // the kept prefix from the threshold's value: no selection
+    cC = (uint64_t)okey(xc) << 32;
+  } else {
+    select_in_bin<DT>(S, ws, row, false, nk);
+    cC = st.su[4];
+  }
+  bar();
+  if (threadIdx.x == 0) {
+    st.su[4] = cC;
+    st.su[5] = nk;
+  }
+  bar();
+}
+// The cut by count (by_mass = 0) or mantissa sum inside row bin rb: its comp -> st.su[4], its inclusive prefix -> st.su[5]
+template <int DT>
+__device__ __noinline__ void rank_cut(QWS_L ResolveLds* s, char* ws_, int row_, int rb_, int by_mass_, uint64_t target_) {
+  ResolveLds& S = *(ResolveLds*)s;
+  char* const ws = uniform_ptr(ws_);
+  const int row = __builtin_amdgcn_readfirstlane(row_), rb = __builtin_amdgcn_readfirstlane(rb_);
+  const bool by_mass = __builtin_amdgcn_readfirstlane(by_mass_) != 0;
+  const uint64_t target = readlane<uint64_t>(target_, 0);
+  RS& st = S.st;
+  uint64_t c = ~0ull, pref = 0;
+  if (!select_listed<DT>(S, ws, row, rb, by_mass, target, &c, &pref)) {
+    gather<DT>(S, ws, row, rb);
+    select_in_bin<DT>(S, ws, row, by_mass, target);
+    c = st.su[4];
+    pref = st.su[5];
+  }
+  bar();
+  if (threadIdx.x == 0) {
+    st.su[4] = c;
+    st.su[5] = pref;
+  }
+  bar();
+}
+// The mantissa sum of the gathered bin's candidates with comp >= cmin -> st.su[7]
+template <int DT>
+__device__ __noinline__ void bin_mass(QWS_L ResolveLds* s, char* ws, int row, uint64_t cmin) {
+  ResolveLds& S = *(ResolveLds*)s;
+  unsigned long long v = 0;
+  for_bin<DT>(S, uniform_ptr(ws), __builtin_amdgcn_readfirstlane(row), [&](uint64_t c, uint32_t mu) { v += c >= cmin ? (unsigned long long)mu : 0ull; });
+  block_add_u64(S.st, v);
+}
+// Adds the gathered bin's kept candidates (comp >= cC) to the blocks' kept masses
+template <int DT>
+__device__ __noinline__ void kept_unstaged(QWS_L ResolveLds* s, char* ws, int row, uint64_t cC, int sh_) {
+  ResolveLds& S = *(ResolveLds*)s;
+  const int sh = __builtin_amdgcn_readfirstlane(sh_);
+  for_bin<DT>(S, uniform_ptr(ws), __builtin_amdgcn_readfirstlane(row), [&](uint64_t c, uint32_t mu) {
+    if (c >= cC) {
+      const int g = (int)(comp_idx(c) / BLK);
+      atomic_add_u128(&S.st.Klo[g], &S.st.Khi[g], (u128)mu << sh);
+    }
+  });
+}
+// Dense probabilities of the kept set, by rescans of every block (k_scan has written zeros)
+template <int DT>
+__device__ __noinline__ void dense_probs(QWS_L ResolveLds* s, char* ws_, int row_, unsigned long long s2lo, unsigned long long s2hi, int cR_, uint64_t cC_) {
+  using BL = Blk<DT, NT2>;
+  ResolveLds& S = *(ResolveLds*)s;
+  char* const ws = uniform_ptr(ws_);
+  const int row = __builtin_amdgcn_readfirstlane(row_), cR = __builtin_amdgcn_readfirstlane(cR_);
+  const uint64_t cC = readlane<uint64_t>(cC_, 0);
+  const double S2d = (double)s2hi * 18446744073709551616.0 + (double)s2lo;
+  const int G = __builtin_amdgcn_readfirstlane(S.st.G), V = S.B.V, row_top = S.st.row_top;
+  const float K = S.st.K;
+  float* out = S.B.out_probs + (size_t)row * V;
+  for (int g = 0; g < G; g++) {
+    if (__builtin_amdgcn_readfirstlane(S.bi[g].dn) < 0) continue;
+    stage_block<DT>(s, ws, row, g);
+    const float* xs = (const float*)S.big;
+    const int t0 = (int)threadIdx.x * BL::EPT;
+#pragma unroll
+    for (int k = 0; k < BL::EPT; k++) {
+      const float v = xs[big_at(t0) + k];
+      if (v == -INFINITY) continue;
+      const W w = weigh(tval(v, K), S.ts);
+      const int r = row_top - w.bin();
+      const uint32_t idx = (uint32_t)(g * BLK + t0 + k);
+      if (r < NR && (r < cR || (r == cR && comp(okey(v), idx) >= cC))) out[idx] = (float)((double)rw1(w.mu, r) / S2d);
+    }
+    bar();
+  }
 }
 
 // VER: the rows of a verify call (rres != nullptr)
 template <int DT, bool VER>
 __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, RowRes* rres) {
-  __shared__ __attribute__((aligned(16))) unsigned long long s_fb[MAXG * FB];
-  __shared__ unsigned long long s_emu[MAXG * NEXP];
-  __shared__ uint64_t s_ec[XG];
-  __shared__ uint32_t s_em[XG];
-  __shared__ __attribute__((aligned(16))) uint32_t s_big[BIGW];
-  __shared__ int s_nt;
-  __shared__ __attribute__((aligned(16))) float2 s_ts[1024];
-  __shared__ BI s_bi[MAXG];
-  __shared__ RS s_st;
-  __shared__ u128 s_red[NWV2 + 1];
-  RL L;
-  L.bi = s_bi;
-  L.st = &s_st;
-  L.ts = s_ts;
-  L.big = s_big;
-  L.fb = s_fb;
-  L.emu = s_emu;
-  L.ec = s_ec;
-  L.em = s_em;
-  L.nt = &s_nt;
-  L.red = s_red;
-  __shared__ qws_batch s_B;  // LDS copies the non-inlined block stager reads
-  __shared__ qws_row s_R;
-  RS& st = s_st;
+  __shared__ __attribute__((aligned(16))) ResolveLds S;
+  QWS_L ResolveLds* const SL = (QWS_L ResolveLds*)&S;
+  const RL L = rl_of(S);
+  auto& s_fb = S.fb;
+  auto& s_emu = S.emu;
+  auto& s_bi = S.bi;
+  RS& st = S.st;
   // Workgroup i runs on XCD i % 8 (round-robin dispatch): it takes a row whose blocks k_scan ran on that XCD (rows
   // [x * RB, (x + 1) * RB) there, RB = ceil(B / 8)), so the row's records are read back through the L2 that wrote them.
   const int RB = (B.B + NXCD - 1) / NXCD;
@@ -1573,13 +1725,13 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
   if (tid < 512) tv = gmem((const vu4*)EXP2_TS)[tid];
   const qws_row R = B.rows[row];
   if (tid == 0) {
-    s_B = B;
-    s_R = R;
+    S.B = B;
+    S.R = R;
   }
-  const qws_batch& BB = s_B;
-  const qws_row& RR = s_R;
+  const qws_batch& BB = S.B;
+  const qws_row& RR = S.R;
   const uint32_t u_draw = draw_u24(R.seed, R.position, R.stream, R.row_key, R.draw_word);  // the draw's Philox word
-  if (tid < 512) ((vu4*)s_ts)[tid] = tv;
+  if (tid < 512) ((vu4*)S.ts)[tid] = tv;
 #pragma unroll
   for (int k = 0; k < HPT; k++) {
     const int i = tid + k * NT2;
@@ -1601,12 +1753,12 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
     st.fxn = 0;
   }
   bar();
+  __shared__ TopRow s_top;
   if (listed_top(R)) {  // uniform
-    __shared__ TopRow s_top;
-    if (tid == 0) s_top = TopRow{row, B.V, G, R.top_k, u_draw, R.temperature, R.top_p, R.min_p, R.log2_min_p, B.out_tokens, B.out_info, B.out_probs, rres};
+    if (tid == 0) s_top = TopRow{row, B.V, G, R.top_k, u_draw, R.temperature, R.top_p, R.min_p, R.log2_min_p, 0, 0, B.out_tokens, B.out_info, B.out_probs, rres};
     bar();
-    const int tk = resolve_top<VER>((QWS_L const TopRow*)&s_top, (QWS_L const char*)s_fb, (QWS_L const float2*)s_ts, (QWS_L char*)s_big);
-    if (!VER && B.advance) advance_row(B, R, row, tk, &s_nt, -1, 0, 0u);
+    const int tk = resolve_top<VER>((QWS_L const TopRow*)&s_top, (QWS_L const char*)s_fb, (QWS_L const float2*)S.ts, (QWS_L char*)S.big);
+    if (!VER && B.advance) advance_row(B, R, row, tk, &S.nt, -1, 0, 0u);
     return;
   }
   auto hdr = [&](int g) -> const Rec& { return *(const Rec*)((const char*)s_fb + (size_t)g * HDR_BYTES); };
@@ -1649,7 +1801,7 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
       }
     }
     // a row without a candidate emits token 0 (its greedy token) and takes the step with it, as qws_finish_rows does
-    if (!VER && B.advance) advance_row(B, R, row, best == 0 ? 0 : (int)comp_idx(best), &s_nt, -1, 0, 0u);
+    if (!VER && B.advance) advance_row(B, R, row, best == 0 ? 0 : (int)comp_idx(best), &S.nt, -1, 0, 0u);
     return;
   }
   const float tmax = tval(okey_val(comp_key(best)), K);
@@ -1685,45 +1837,75 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
   before_bin(L, NR, &mb, &kept_n);
   // candidates below the row's window (weight 0) still count for top-k: the window's count is a lower bound, and a
   // K at or beyond it keeps every weighted candidate
-  auto bin_kept = [&](uint64_t cmin, bool by_mass) -> unsigned long long {  // kept count / mantissa sum of the gathered bin
-    unsigned long long v = 0;
-    for_bin<DT>(L, BB, RR, ws, row, [&](uint64_t c, uint32_t mu) {
-      if (c >= cmin) v += by_mass ? (unsigned long long)mu : 1ull;
-    });
-    block_add_u64(st, v);
-    return st.su[7];
+  // ---- at most 64 candidates down to row bin rb (NR: all that weigh something; else rb's power is the staged one), all in
+  // their blocks' lists (each block's bins from its best down to rb's listed): they are taken from the lists and the row
+  // is finished over them, with no selection inside a bin, no other power staged, no kept masses per block and no block
+  // of the draw.  thr: the top-p threshold when the row's mass is known (0: min-p, then top-p over the candidates'
+  // own mass).  Test flags that ask for rescans or staged draws keep the general path.
+  auto small = [&](int rb, u128 thr) -> bool {
+    if (R.test_flags & (QWS_TF_RESCAN | QWS_TF_STAGED_DRAW | QWS_TF_SPLIT_SELECT)) return false;
+    const int lane = lane_id();
+    int cnt = 0;
+    bool ok = true;
+    if (lane < G && s_bi[lane].dn >= 0) {
+      const BI& b = s_bi[lane];
+      if (rb >= NR) {
+        cnt = b.wcnt;
+        ok = cnt == 0 || (b.w0 == 0 && cnt <= b.n_list);
+      } else {
+        const int cb = rb - FB * b.dn;  // the bin among the block's own
+        const int r0 = b.c * FB + (FB - 1) - (tfloor(tval(okey_val(b.max_key), K)) >> 4);  // its best's
+        if (cb >= r0) {
+          if (cb < b.nbw) {
+            const unsigned long long wd = s_fb[lane * FB + (rb & 63)];
+            ok = b.w0 == 0 && bw_listed(wd);
+            cnt = (int)(bw_off(wd) + bw_cnt(wd));
+          } else {  // past its last occupied bin (with a top-k cut the bins may end earlier)
+            ok = b.w0 == 0 && b.w1 >= b.nbw - 1 && R.top_k <= 0;
+            cnt = b.n_list;
+          }
+        }
+      }
+    }
+    const int inc = wave_scan_incl<int>(cnt), tot = readlane<int>(inc, 63), exc = inc - cnt;
+    if (__ballot(!ok) != 0ull || tot > 64 || tot == 0) return false;  // uniform: the same words in every wave
+    TopBuf& T = *(TopBuf*)S.big;
+    if (wave_id() == 0) {
+      // list entry `lane` of the concatenation: its block by a binary search over the inclusive counts
+      int g = 0;
+      for (int sft = 32; sft > 0; sft >>= 1) g += __shfl(inc, g + sft - 1) <= lane ? sft : 0;
+      const int e0 = __shfl(exc, min(g, 63));
+      T.lst[lane] = lane < tot ? els_of(ws, G, row, g)[lane - e0] : 0ull;
+      if (lane == 0)
+        s_top = TopRow{row, B.V, G, 64, u_draw, R.temperature, R.top_p, thr == 0 ? R.min_p : 0.0f, R.log2_min_p, (unsigned long long)thr,
+                       (unsigned long long)(thr >> 64), B.out_tokens, B.out_info, B.out_probs, rres};
+    } else if (wave_id() == 1) {
+      T.lst[64 + lane] = 0ull;
+    }
+    bar();
+    const int tk = finish_small<VER>((QWS_L const TopRow*)&s_top, tot, (QWS_L const float2*)S.ts, (QWS_L char*)S.big);
+    if (tid == 0 && B.out_info && tk >= 0 && st.rescans) B.out_info[row] = 1;
+    if (!VER && B.advance) advance_row(B, R, row, tk, &S.nt, -1, 0, 0u);
+    return true;
   };
   if (R.min_p > 0.0f) {
     const float tcut = (float)((double)(tmax / 1024.0f) + R.log2_min_p) * 1024.0f;
     const int rc = row_top - (tfloor(tcut) >> 4);
     bool need = rc < NR;
-    if (need && R.top_k > 0) {  // uniform: top_k candidates in the bins above the min-p cut's: the top-k cut decides
-      stage_power(L, ws, row, rc >> 6);
-      u128 mass_unused;
-      unsigned long long above;
-      before_bin(L, rc, &mass_unused, &above);
-      need = above < (unsigned long long)R.top_k;
-    }
     if (need) {
       stage_power(L, ws, row, rc >> 6);
-      gather<DT, VER>(L, BB, RR, ws, row, rc);
-      // kept: t >= tcut, a prefix of the bin in comp order
-      unsigned long long v = 0;
-      for_bin<DT>(L, BB, RR, ws, row, [&](uint64_t c, uint32_t) { v += tval(okey_val(comp_key(c)), K) >= tcut ? 1ull : 0ull; });
-      block_add_u64(st, v);
-      const unsigned long long nk = st.su[7];
+      if (small(rc, 0)) return;  // uniform
+    }
+    if (need && R.top_k > 0) {  // uniform: top_k candidates in the bins above the min-p cut's: the top-k cut decides
+      const int lane = lane_id();
+      const uint32_t above = wave_sum<uint32_t>((lane < (rc >> 6) ? st.Rc[lane] : 0u) + (lane < (rc & 63) ? st.fcnt[lane] : 0u));
+      need = above < (uint32_t)R.top_k;
+    }
+    if (need) {
+      minp_cut<DT>(SL, ws, row, rc, tcut);
       cR = rc;
-      float xc;
-      if (nk == 0) {
-        cC = ~0ull;
-      } else if (nk == (unsigned long long)st.gn) {
-        cC = 0;
-      } else if (first_x_t(tcut, K, &xc)) {  // the kept prefix from the threshold's value: no selection
-        cC = (uint64_t)okey(xc) << 32;
-      } else {
-        select_in_bin<DT>(L, BB, RR, ws, row, false, nk);
-        cC = st.su[4];
-      }
+      cC = st.su[4];
+      const unsigned long long nk = st.su[5];
       before_bin(L, rc, &mb, &kept_n);
       kept_n += nk;
     }
@@ -1740,136 +1922,44 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
     const int bk = pk * FB + fine_cross(L, false, (u128)before_p, (u128)(unsigned long long)R.top_k, &before_f);
     const unsigned long long need = (unsigned long long)R.top_k - (unsigned long long)before_f;
     cR = bk;
-    uint64_t pref_unused;
     if (st.fcnt[bk & 63] == need) {  // the whole bin is kept (cC = 0): no gather
       cC = 0;
-    } else if (!select_listed<DT>(L, BB, RR, ws, row, bk, false, need, &cC, &pref_unused)) {
-      gather<DT, VER>(L, BB, RR, ws, row, bk);
-      select_in_bin<DT>(L, BB, RR, ws, row, false, need);
+    } else {
+      rank_cut<DT>(SL, ws, row, bk, 0, need);
       cC = st.su[4];
     }
   }
-  // ---- a cut set (min-p / top-k) of at most 64 candidates, all in their blocks' lists (each block's bins from its top
-  // down to the cut listed without a gap): wave 0 holds them, one per lane, and finishes the row -- the top-p cut over
-  // their exact weights in value order, then the draw in index order -- with no other power staged, no kept masses
-  // per block and no block of the draw.  The same definition as the path below; test flags that ask for rescans or
-  // staged draws keep that path.
-  const unsigned long long n_cut = (R.top_k > 0 && (unsigned long long)R.top_k <= kept_n) ? (unsigned long long)R.top_k : kept_n;
-  __shared__ int s_fast, s_ftok, s_fcR;
-  __shared__ unsigned long long s_fS[2], s_fcC;
+  if (cR == NR && kept_n <= 64 && small(NR, 0)) return;  // uniform: no cut so far (a few strongly biased tokens, say)
   u128 S2;
   int tok = -1;
-  bool fast = false;
-  if (cR < NR && n_cut > 0 && n_cut <= 64 && st.fpow == (cR >> 6) &&
-      !(R.test_flags & (QWS_TF_RESCAN | QWS_TF_STAGED_DRAW | QWS_TF_SPLIT_SELECT))) {  // uniform
-    if (wave_id() == 0) {
-      const int lane = lane_id();
-      // lane g: the number of block g's list entries in its bins down to the cut's (bins 0 .. cb listed, no gap)
-      int cnt = 0;
-      bool ok = true;
-      if (lane < G && s_bi[lane].dn >= 0) {
-        const BI& b = s_bi[lane];
-        const int cb = cR - FB * b.dn;  // the cut's bin among the block's own
-        if (cb >= 0) {
-          const unsigned long long wd = s_fb[lane * FB + (cR & 63)];
-          ok = cb < b.nbw && b.w0 == 0 && cb <= b.w1 && bw_listed(wd);
-          cnt = ok ? (int)(bw_off(wd) + bw_cnt(wd)) : 0;
-        }
-      }
-      const int inc = wave_scan_incl<int>(cnt), tot = readlane<int>(inc, 63), exc = inc - cnt;
-      int res = 0;
-      if (__ballot(!ok) == 0ull && tot <= 64) {  // uniform in the wave
-        // list entry `lane` of the concatenation: its block by a binary search over the inclusive counts (all lanes)
-        int g = 0;
-        for (int sft = 32; sft > 0; sft >>= 1) g += __shfl(inc, g + sft - 1) <= lane ? sft : 0;
-        const int e0 = __shfl(exc, min(g, 63));
-        uint64_t c = 0, w = 0;
-        uint32_t idx = 0xFFFFFFFFu;
-        int r = NR;
-        if (lane < tot) {
-          c = els_of(ws, G, row, g)[lane - e0];
-          const float t = tval(okey_val(comp_key(c)), K);
-          r = row_top - (tfloor(t) >> 4);
-          if (r < cR || (r == cR && c >= cC)) w = rw1(weigh(t, L.ts).mu, r);
-          idx = comp_idx(c);
-        }
-        if ((unsigned long long)__popcll(__ballot(w != 0)) == n_cut) {  // every kept candidate is here
-          const u128 S = wave_sum_u128((u128)w);
-          u128 s2 = S;
-          uint64_t cK = cC;
-          int rK = cR;
-          uint64_t wk = w;  // the kept weight after top-p
-          if (R.top_p < 1.0f) {
-            const uint64_t TP = (uint64_t)floor((double)R.top_p * 4294967296.0);
-            const u128 thr = mul_shr_ceil(S, TP, 32);
-            if (thr > 0) {
-              u128 above = 0;  // kept weight of the larger comps
-              for (int j = 0; j < tot; j++) {  // uniform
-                const uint64_t cj = readlane<uint64_t>(c, j), wj = readlane<uint64_t>(w, j);
-                above += cj > c ? (u128)wj : (u128)0;
-              }
-              const int k = min(first_lane(w != 0 && above < thr && thr <= above + w), 63);  // thr <= S: one lane crosses
-              cK = readlane<uint64_t>(c, k);
-              rK = readlane<int>(r, k);
-              s2 = readlane<u128>(above + w, k);
-              wk = c >= cK ? w : 0;
-            }
-          }
-          const u128 tt = mul_shr_floor(s2, u_draw, 24);
-          u128 below = 0;  // kept weight of the lower indices
-          for (int j = 0; j < tot; j++) {  // uniform
-            const uint32_t ij = readlane<uint32_t>(idx, j);
-            const uint64_t wj = readlane<uint64_t>(wk, j);
-            below += ij < idx ? (u128)wj : (u128)0;
-          }
-          const int l = first_lane(wk != 0 && below <= tt && tt < below + wk);
-          if (lane == 0) {
-            s_ftok = l < 64 ? (int)readlane<uint32_t>(idx, l) : -1;
-            s_fcR = rK;
-            s_fcC = cK;
-            s_fS[0] = (unsigned long long)s2;
-            s_fS[1] = (unsigned long long)(s2 >> 64);
-          }
-          res = 1;
-        }
-      }
-      if (lane == 0) s_fast = res;
-    }
-    bar();
-    fast = s_fast != 0;
-    if (fast) {
-      tok = s_ftok;
-      cR = s_fcR;
-      cC = s_fcC;
-      S2 = ld128(s_fS[0], s_fS[1]);
-    }
-  }
   int a_g = -1, a_n = 0;  // advance: the drawn block and its state entries, loaded before the draw
   uint32_t a_e = 0u;
-  if (!fast) {
+  {
     bool kept_done = false;  // the kept mass of every block computed with the cut (topp_cut_fast)
     // cC = 0: every element of bin cR is kept, and the bin's words give its mass (the staged power is cR's)
-    u128 S = mb;
+    u128 Sm = mb;  // the row's mass (after min-p and top-k)
     if (cR < NR) {
       unsigned long long cnt_unused;
       before_bin(L, cR, &mb, &cnt_unused);
-      S = mb + shl128(cC == 0 ? st.fmu[cR & 63] : bin_kept(cC, true), D_EXP - (cR >> 6));
+      if (cC != 0) bin_mass<DT>(SL, ws, row, cC);
+      Sm = mb + shl128(cC == 0 ? st.fmu[cR & 63] : st.su[7], D_EXP - (cR >> 6));
     }
     if (R.top_p < 1.0f) {
       const uint64_t TP = (uint64_t)floor((double)R.top_p * 4294967296.0);
-      const u128 thr = mul_shr_ceil(S, TP, 32);
+      const u128 thr = mul_shr_ceil(Sm, TP, 32);
       if (thr > 0) {
         int pp;
         u128 before_p, before_f;
         pow_cross_mass(L, thr, &pp, &before_p);
         stage_power(L, ws, row, pp);
         const int bp = pp * FB + fine_cross(L, true, before_p, thr, &before_f);
+        if (small(bp, thr)) return;  // uniform
         const int sh = D_EXP - pp;
         cR = bp;
         mb = before_f;
         if (st.fcnt[bp & 63] == 1) {  // the crossing bin holds one element: the cut, the whole bin kept (no gather)
           cC = 0;
-          S = mb + ((u128)st.fmu[bp & 63] << sh);
+          Sm = mb + ((u128)st.fmu[bp & 63] << sh);
         } else {
           // the crossing in mantissa units of the bin's power: sum of mu * 2^sh >= thr - before  <=>  sum of mu >= ceil(...)
           const u128 need = thr - before_f;
@@ -1877,17 +1967,16 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
           uint64_t pref;  // the selection's inclusive mantissa sum at the cut
           if (topp_cut_fast(L, RR, ws, row, bp, tmu, &cC, &pref)) {
             kept_done = true;
-          } else if (!select_listed<DT>(L, BB, RR, ws, row, bp, true, tmu, &cC, &pref)) {
-            gather<DT, VER>(L, BB, RR, ws, row, bp);
-            select_in_bin<DT>(L, BB, RR, ws, row, true, tmu);
+          } else {
+            rank_cut<DT>(SL, ws, row, bp, 1, tmu);
             cC = st.su[4];
             pref = st.su[5];
           }
-          S = mb + ((u128)pref << sh);
+          Sm = mb + ((u128)pref << sh);
         }
       }
     }
-    S2 = S;
+    S2 = Sm;
     // a verify row ends at S2: the verify kernels draw from p for the one row of a sequence that needs it
     if constexpr (!VER) {
       // ---- kept mass per block: its powers above the cut's, its fine bins above the cut's bin and its kept elements there
@@ -1904,7 +1993,7 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
             for (int f = j; f < (cR & 63) + (cC == 0 ? 1 : 0); f += 16) k += shl128(bw_mu(s_fb[g * FB + f]), sh);
             if (cC != 0 && st.gstaged) {  // a partial cut: the gathered bin is cR's
               for (int i = b.gofs + j; i < b.gofs + (b.gsrc ? b.gcnt : 0); i += 16)
-                if (s_ec[i] >= cC) k += (u128)s_em[i] << sh;
+                if (L.ec[i] >= cC) k += (u128)L.em[i] << sh;
             }
           }
         }
@@ -1915,15 +2004,8 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
         }
       }
       if (!kept_done) bar();
-      if (!kept_done && cR < NR && cC != 0 && !st.gstaged) {  // a bin too large for LDS: its kept elements by block from the sources
-        const int sh = D_EXP - (cR >> 6);
-        for_bin<DT>(L, BB, RR, ws, row, [&](uint64_t c, uint32_t mu) {
-          if (c >= cC) {
-            const int g = (int)(comp_idx(c) / BLK);
-            atomic_add_u128(&st.Klo[g], &st.Khi[g], (u128)mu << sh);
-          }
-        });
-      }
+      // a bin too large for LDS: its kept elements by block from the sources
+      if (!kept_done && cR < NR && cC != 0 && !st.gstaged) kept_unstaged<DT>(SL, ws, row, cC, D_EXP - (cR >> 6));
       // ---- the draw: the block by its kept mass (index order), then the token inside it
       const u128 tt = mul_shr_floor(S2, u_draw, 24);
       int gs;   // every wave picks it from the final kept masses (no barrier)
@@ -1967,29 +2049,10 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
       }
     }
   }
-  if (B.out_probs) {  // dense probabilities of the kept set (test-hook path), by rescans of every block
-    using BL = Blk<DT, NT2>;
-    const double S2d = (double)(uint64_t)(S2 >> 64) * 18446744073709551616.0 + (double)(uint64_t)S2;
-    for (int g = 0; g < G; g++) {
-      if (s_bi[g].dn < 0) continue;
-      stage_block<DT>(L, BB, RR, ws, row, g);
-      const float* xs = (const float*)s_big;
-      const int t0 = tid * BL::EPT;
-#pragma unroll
-      for (int k = 0; k < BL::EPT; k++) {
-        const float v = xs[big_at(t0) + k];
-        if (v == -INFINITY) continue;
-        const W w = weigh(tval(v, K), s_ts);
-        const int r = row_top - w.bin();
-        const uint32_t idx = (uint32_t)(g * BLK + t0 + k);
-        if (r < NR && (r < cR || (r == cR && comp(okey(v), idx) >= cC))) B.out_probs[(size_t)row * B.V + idx] = (float)((double)rw1(w.mu, r) / S2d);
-      }
-      bar();
-    }
-  }
+  if (B.out_probs) dense_probs<DT>(SL, ws, row, (unsigned long long)S2, (unsigned long long)(S2 >> 64), cR, cC);  // uniform
   if (tid == 0) {
     B.out_tokens[row] = tok;
-    if (B.out_info) B.out_info[row] = tok < 0 && (fast || !VER) ? -1 : (st.rescans ? 1 : 0);
+    if (B.out_info) B.out_info[row] = tok < 0 && !VER ? -1 : (st.rescans ? 1 : 0);
     if (VER) {
       RowRes o;
       o.s_lo = (unsigned long long)S2;
@@ -1998,7 +2061,7 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
       o.cR = cR;
       o.row_top = row_top;
       o.K = K;
-      o.kind = tok < 0 && fast ? RR_FAIL : RR_SAMPLED;  // outside the one-wave finish tok = -1: not drawn here
+      o.kind = RR_SAMPLED;  // tok = -1: not drawn here
       o.tok = tok;
       o.pad = 0;
       rres[row] = o;
@@ -2008,7 +2071,7 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
     __shared__ int s_tok;
     if (tid == 0) s_tok = tok;  // thread 0 holds the row's token (a listed draw leaves it in wave 0 only)
     bar();
-    advance_row(B, R, row, s_tok, &s_nt, a_g, a_n, a_e);
+    advance_row(B, R, row, s_tok, &S.nt, a_g, a_n, a_e);
   }
 }
 
