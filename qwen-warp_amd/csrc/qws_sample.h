@@ -121,40 +121,6 @@ __device__ __forceinline__ T top_bound(F key, T lo, int need, int enough, int* n
   return lo;
 }
 
-// ---------------------------------------------------------------------------------------------- block searches
-// Wave-level searches over a block's LDS histogram (hist[rel] = count << 40 | mantissa sum) and its per-power sums,
-// by all 64 lanes of one wave: first the power of two, then the fine bin inside it.
-// Inclusive cumulative count up to bin r (0 for r < 0)
-__device__ inline uint32_t blk_cnt_to(const unsigned long long* hist, const uint32_t* ecnt, int r) {
-  if (r < 0) return 0u;
-  r = min(r, NBIN - 1);
-  const int lane = lane_id(), p = r >> 6;
-  uint32_t v = lane < p ? ecnt[lane] : 0u;
-  v += lane <= (r & 63) ? (uint32_t)(hist[p * FB + lane] >> 40) : 0u;
-  return wave_sum<uint32_t>(v);
-}
-// approximate mass (relative to the block's top power of two) up to bin r
-__device__ inline float blk_mass_to(const unsigned long long* hist, const unsigned long long* emu, int r) {
-  if (r < 0) return 0.0f;
-  r = min(r, NBIN - 1);
-  const int lane = lane_id(), p = r >> 6;
-  float v = lane < p ? ldexpf((float)emu[lane], -lane) : 0.0f;
-  v += lane <= (r & 63) ? ldexpf((float)(hist[p * FB + lane] & M40), -p) : 0.0f;
-  return wave_sum<float>(v);
-}
-// first bin whose inclusive cumulative count reaches tgt (NBIN when none)
-__device__ inline int blk_cross_cnt(const unsigned long long* hist, const uint32_t* ecnt, uint32_t tgt) {
-  const int lane = lane_id();
-  const uint32_t pc = lane < NEXP ? ecnt[lane] : 0u;
-  const uint32_t inc = wave_scan_incl<uint32_t>(pc);
-  const int p = first_lane(lane < NEXP && inc >= tgt);
-  if (p >= NEXP) return NBIN;
-  const uint32_t base = readlane<uint32_t>(inc - pc, p);
-  const uint32_t fi = wave_scan_incl<uint32_t>((uint32_t)(hist[p * FB + lane] >> 40)) + base;
-  const int f = first_lane(fi >= tgt);
-  return p * FB + min(f, 63);
-}
-
 // ---------------------------------------------------------------------------------------------- k_resolve
 // One workgroup per row.  Global loads come in few parallel rounds (the headers; the fine bins of one power of two of
 // every block; one bin's listed elements; the block of the draw); everything else runs from LDS.

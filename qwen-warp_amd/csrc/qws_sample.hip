@@ -262,17 +262,20 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
   bar();
   float M = s_redf[0];
   for (int i = 1; i < NWV1; i++) M = fmaxf(M, s_redf[i]);
-  if (M != -INFINITY && mloc == M) {  // equal values compare equal across -0 / +0
-    uint32_t im = 0xFFFFFFFFu;
-#pragma unroll
-    for (int e = EPT - 1; e >= 0; e--)
-      if (x[e] == M) im = (uint32_t)(lo + BL::local(e));
-    atomicMin(&s_imin, im);
-  }
   const float K = kscale(R.temperature);
   const bool samp = R.temperature > 0.0f && K < INFINITY;
-  bar();
-  const uint32_t imax = s_imin;
+  uint32_t imax = 0u;  // the best's lowest index: a greedy row's token (a sampled row's best gives its top power alone)
+  if (!samp) {  // uniform
+    if (M != -INFINITY && mloc == M) {  // equal values compare equal across -0 / +0
+      uint32_t im = 0xFFFFFFFFu;
+#pragma unroll
+      for (int e = EPT - 1; e >= 0; e--)
+        if (x[e] == M) im = (uint32_t)(lo + BL::local(e));
+      atomicMin(&s_imin, im);
+    }
+    bar();
+    imax = s_imin;
+  }
   bool below = false;  // the block's best more than D_EXP powers of two below the biased tokens' bound
   int dlb = 0;         // powers of two from the block's best up to the bound (when below it)
   if (lbrow && samp && M != -INFINITY) {  // uniform
@@ -347,26 +350,24 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
     }
   }
   bar();
-  // ---- exact counts and mantissa sums per power of two (eight threads per power, eight bins each), and the last
-  // occupied bin (s_relmin, 0 before)
+  // ---- exact counts and mantissa sums per power of two (eight threads per power, every eighth bin each: consecutive
+  // lanes read consecutive bins; summed over the eight lanes by DPP), and the last occupied bin (s_relmin, 0 before)
   if (tid < NEXP * 8) {
-    const int b0 = (tid >> 3) * FB + (tid & 7) * 8;
+    const int b0 = (tid >> 3) * FB + (tid & 7);
+    unsigned long long h[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) h[k] = hist[b0 + 8 * k];
     uint32_t cn = 0, last = 0;
     unsigned long long mu = 0;
 #pragma unroll
     for (int k = 0; k < 8; k++) {
-      const unsigned long long h = hist[b0 + k];
-      cn += (uint32_t)(h >> 40);
-      mu += h & M40;
-      last = h ? (uint32_t)(b0 + k) : last;
+      cn += (uint32_t)(h[k] >> 40);
+      mu += h[k] & M40;
+      last = h[k] ? (uint32_t)(b0 + 8 * k) : last;
     }
-#pragma unroll
-    for (int m = 1; m < 8; m <<= 1) {
-      cn += (uint32_t)__shfl_xor((int)cn, m);
-      const uint32_t lo32 = (uint32_t)__shfl_xor((int)(uint32_t)mu, m), hi32 = (uint32_t)__shfl_xor((int)(uint32_t)(mu >> 32), m);
-      mu += ((unsigned long long)hi32 << 32) | lo32;
-      last = max(last, (uint32_t)__shfl_xor((int)last, m));
-    }
+    cn = sum8<uint32_t>(cn);
+    mu = sum8<unsigned long long>(mu);
+    last = max8(last);
     if ((tid & 7) == 0) {
       s_ecnt[tid >> 3] = cn;
       s_emu[tid >> 3] = mu;
@@ -379,41 +380,61 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
   // ---- wave 0: the bins to write (down to the deepest bin a row cut can reach here: the block's own min-p cut and
   // its own K-th candidate, since the row's are at or above them) and the window of listed bins
   if (wave == 0) {
+    // power-level inclusive prefixes: counts (exact) and approximate masses (relative to the block's top power)
+    const uint32_t pcn = lane < NEXP ? s_ecnt[lane] : 0u;
+    const float pms = lane < NEXP ? ldexpf((float)s_emu[lane], -lane) : 0.0f;
+    const uint32_t icn = wave_scan_incl<uint32_t>(pcn);
+    const float ims = wave_scan_incl<float>(pms);
+    // the count through bin r >= 0
+    auto cnt_to = [&](int r) -> uint32_t {
+      const int p = r >> 6;
+      const uint32_t v = wave_sum<uint32_t>(lane <= (r & 63) ? (uint32_t)(hist[p * FB + lane] >> 40) : 0u);
+      return v + (p > 0 ? readlane<uint32_t>(icn, p - 1) : 0u);
+    };
+    auto mass_to = [&](int r) -> float {  // the approximate mass through it
+      const int p = r >> 6;
+      const float v = wave_sum<float>(lane <= (r & 63) ? ldexpf((float)(hist[p * FB + lane] & M40), -p) : 0.0f);
+      return v + (p > 0 ? readlane<float>(ims, p - 1) : 0.0f);
+    };
+    // the first bin whose inclusive count reaches tgt (NBIN: none); *through = that count
+    auto cross_cnt = [&](uint32_t tgt, uint32_t* through) -> int {
+      const int p = first_lane(lane < NEXP && icn >= tgt);
+      if (p >= NEXP) return NBIN;
+      const uint32_t fi = wave_scan_incl<uint32_t>((uint32_t)(hist[p * FB + lane] >> 40)) + (p > 0 ? readlane<uint32_t>(icn, p - 1) : 0u);
+      const int f = min(first_lane(fi >= tgt), 63);
+      *through = readlane<uint32_t>(fi, f);
+      return p * FB + f;
+    };
     int floor_r = NBIN - 1, hard = NBIN - 1;
+    uint32_t thr_unused;
     if (minp) {
       const float tcut = (float)((double)(tval(M, K) / 1024.0f) + R.log2_min_p) * 1024.0f;
       const int rm = btop - (((int)floorf(tcut)) >> 4);
       if (rm < NBIN) floor_r = hard = max(rm, 0);
     }
     if (topk) {
-      hard = min(hard, blk_cross_cnt(hist, s_ecnt, (uint32_t)R.top_k));
+      hard = min(hard, cross_cnt((uint32_t)R.top_k, &thr_unused));
       // the block's likely share of the row's top K (the resolver checks that its window holds the row's cut)
       const uint32_t kk = R.top_k <= 64 ? (uint32_t)R.top_k : (uint32_t)min(R.top_k, 2 * R.top_k / G + 64);
-      floor_r = min(floor_r, blk_cross_cnt(hist, s_ecnt, kk));
+      floor_r = min(floor_r, cross_cnt(kk, &thr_unused));
     }
     floor_r = min(floor_r, r1);
     int w0 = 1, w1 = 0;
-    // power-level inclusive prefixes: counts (exact) and approximate masses (relative to the block's top power); when
-    // floor_r is the last occupied bin the block's totals cover it
-    const uint32_t pcn = lane < NEXP ? s_ecnt[lane] : 0u;
-    const float pms = lane < NEXP ? ldexpf((float)s_emu[lane], -lane) : 0.0f;
-    const uint32_t icn = wave_scan_incl<uint32_t>(pcn);
-    const float ims = wave_scan_incl<float>(pms);
-    const bool at_last = floor_r == r1;
-    bool slots_done = false;  // the list slots already written (a flat top-p window, from the shrink's prefix)
-    uint32_t slots_n = 0;
+    uint32_t before = 0, n_list = 0;  // candidates above w0, and in [w0, w1]
+    const bool at_last = floor_r == r1;  // the block's totals cover it
     if (topk || topp || minp) {
-      const uint32_t nf = at_last ? readlane<uint32_t>(icn, NEXP - 1) : blk_cnt_to(hist, s_ecnt, floor_r);
+      const uint32_t nf = at_last ? readlane<uint32_t>(icn, NEXP - 1) : cnt_to(floor_r);
       if (nf <= (uint32_t)CAP) {  // the whole top set
         w0 = 0;
         w1 = floor_r;
+        n_list = nf;
       } else {
         int b = floor_r;
         bool flat = false;
         if (topp) {
           // the block's own top-p boundary bp (mass crossing) and the power of its (CTOP + 1)-th candidate, both from
           // the power-level prefixes above and one fine-bin scan each (independent: issued together)
-          const float mf = at_last ? readlane<float>(ims, NEXP - 1) : blk_mass_to(hist, s_emu, floor_r);
+          const float mf = at_last ? readlane<float>(ims, NEXP - 1) : mass_to(floor_r);
           const float tm = R.top_p * mf;
           const uint32_t tc = (uint32_t)CTOP + 1u;  // < nf: pC < NEXP
           const int pP = first_lane(lane < NEXP && ims >= tm), pC = first_lane(lane < NEXP && icn >= tc);
@@ -453,14 +474,11 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
             const uint32_t n = wa > wb ? 0u : hi - (ka > 0 ? lo0 : 0u);
             const int kk = first_lane(lane <= span && n <= (uint32_t)CAP);
             const int wl = readlane<int>(wa, kk), wr = readlane<int>(wb, kk);
-            if (wl <= wr) {  // uniform: its slots from the prefix above
+            if (wl <= wr) {  // uniform
               w0 = wl;
               w1 = wr;
-              const uint32_t pb = (uint32_t)__shfl((int)pre, max(lane - 1, 0)), c0 = wl > a0 ? readlane<uint32_t>(pre, wl - a0 - 1) : 0u;
-              const int r = a0 + lane;
-              if (r >= wl && r <= wr) cursor[r] = (lane > 0 ? pb : 0u) - c0;
-              slots_done = true;
-              slots_n = readlane<uint32_t>(pre, wr - a0) - c0;
+              n_list = readlane<uint32_t>(n, kk);
+              if (w0 > 0) before = cnt_to(w0 - 1);
             }
           } else {
             b = min(floor_r, bp + MARGIN_NEAR);
@@ -469,38 +487,26 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
         if (!flat) {  // uniform
           // one range of as many bins as the list holds: from the top when that reaches b (or a min-p floor, which lies
           // higher in the row than in most of its blocks), else the bins ending at b
-          const uint32_t nb = b == floor_r ? nf : blk_cnt_to(hist, s_ecnt, b);
+          const uint32_t nb = b == floor_r ? nf : cnt_to(b);
           if (minp || nb <= (uint32_t)CAP) {
+            uint32_t through;
             w0 = 0;
-            w1 = min(blk_cross_cnt(hist, s_ecnt, (uint32_t)CAP + 1u) - 1, floor_r);
+            w1 = min(cross_cnt((uint32_t)CAP + 1u, &through) - 1, floor_r);  // nf > CAP: the crossing lies at or above floor_r
+            n_list = w1 >= 0 ? cnt_to(w1) : 0u;
           } else {
-            w0 = blk_cross_cnt(hist, s_ecnt, nb - (uint32_t)CAP) + 1;
+            w0 = cross_cnt(nb - (uint32_t)CAP, &before) + 1;
             w1 = b;
+            n_list = nb - before;
           }
         }
-      }
-    }
-    // list slots: a prefix of the listed bins' counts, in rel order (four rounds of 64 bins per step, their counts read
-    // together: a peaked block's range can span hundreds of bins)
-    uint32_t base = slots_n;
-    for (int r0c = w0; r0c <= (slots_done ? -1 : w1); r0c += 256) {  // uniform
-      uint32_t cn[4];
-#pragma unroll
-      for (int j = 0; j < 4; j++) cn[j] = r0c + 64 * j + lane <= w1 ? (uint32_t)(hist[r0c + 64 * j + lane] >> 40) : 0u;
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        if (r0c + 64 * j > w1) break;  // uniform
-        const int r = r0c + 64 * j + lane;
-        const uint32_t inc = wave_scan_incl<uint32_t>(cn[j]);
-        if (r <= w1) cursor[r] = base + inc - cn[j];
-        base += readlane<uint32_t>(inc, 63);
       }
     }
     if (lane == 0) {
       s_win[0] = w0;
       s_win[1] = w1;
-      s_win[4] = (int)base;
+      s_win[4] = (int)n_list;
       s_win[5] = min(r1, hard) + 1;
+      s_win[6] = (int)before;
       s_nl = 0;
     }
   }
@@ -523,12 +529,22 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
     H->emu[tid] = s_emu[tid];
   }
 
+  // a wave writes one power's bin words at a time; a listed bin's slot in the list = the candidates above it from w0 on
+  // (the powers' prefix and one scan inside the power: no wave waits for another's)
   unsigned long long* BW = (unsigned long long*)(rec + BIN_OFF);
-  for (int r = tid; r < nbw; r += NT1) {
+  const uint32_t epc = lane < NEXP ? s_ecnt[lane] : 0u, eex = wave_scan_incl<uint32_t>(epc) - epc - (uint32_t)s_win[6];
+  for (int p = wave; p * FB < nbw; p += NWV1) {  // uniform in the wave
+    const int r = p * FB + lane;
     const unsigned long long h = hist[r];
     unsigned long long wd = (h & M40) | ((h >> 40) << 37);
-    if (r >= w0 && r <= w1) wd |= (1ull << 62) | ((unsigned long long)cursor[r] << 51);
-    BW[r] = wd;
+    if (p * FB <= w1 && p * FB + (FB - 1) >= w0) {  // uniform in the wave
+      const uint32_t cn = (uint32_t)(h >> 40), slot = readlane<uint32_t>(eex, p) + wave_scan_incl<uint32_t>(cn) - cn;
+      if (r >= w0 && r <= w1) {
+        cursor[r] = slot;
+        wd |= (1ull << 62) | ((unsigned long long)slot << 51);
+      }
+    }
+    if (r < nbw) BW[r] = wd;
   }
   if (w0 <= w1) {
     // elements of the listed bins, bucketed by bin: first compacted into LDS as {value bits, local index} (the exp2
