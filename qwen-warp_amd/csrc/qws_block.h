@@ -18,34 +18,54 @@ struct Blk {
   static_assert(EPT % VEC == 0, "whole vectors per thread");
   __device__ static inline int local(int e) { return ((e / VEC) * NTH + (int)threadIdx.x) * VEC + (e % VEC); }
 
-  // Raw logits of block [lo, hi) of `row`, -inf past hi (NaN kept: see fixnan).
-  __device__ static inline void load_raw(const qws_batch& B, int row, int lo, int hi, float (&x)[EPT]) {
+  // A block's logits on the way into x: fp32 logits are loaded there; bf16 logits stay packed (two per word) until
+  // unpack, so that a block waits for its processors' lists in half the registers (unpacked at the load, the
+  // 64-register kernel spilled the mask words behind every load: 32 rows with masks, k_scan 16.8 -> 15.3 us).
+  struct Raw {
+    vu4 v[DT == QWS_DTYPE_F32 ? 1 : S];
+  };
+  // Issues the loads of block [lo, hi) of `row`: -inf past hi (NaN kept: see fixnan).
+  __device__ static inline void load_bits(const qws_batch& B, int row, int lo, int hi, Raw& r, float (&x)[EPT]) {
     const size_t esz = DT == QWS_DTYPE_F32 ? 4 : 2;
     const char* base = (const char*)B.logits + (size_t)row * (size_t)B.row_stride * esz;
 #pragma unroll
     for (int s = 0; s < S; s++) {
       const int i0 = lo + (s * NTH + (int)threadIdx.x) * VEC;
-      if (i0 < hi) {
-        if constexpr (DT == QWS_DTYPE_F32) {
+      if constexpr (DT == QWS_DTYPE_F32) {
+        if (i0 < hi) {
           const vf4 v = *gmem((const vf4*)(base + (size_t)i0 * 4));
           x[s * 4 + 0] = v.x;
           x[s * 4 + 1] = v.y;
           x[s * 4 + 2] = v.z;
           x[s * 4 + 3] = v.w;
         } else {
-          const vu4 v = *gmem((const vu4*)(base + (size_t)i0 * 2));
-          const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-          for (int j = 0; j < 4; j++) {
-            x[s * 8 + 2 * j] = bf16f((uint16_t)(w[j] & 0xFFFFu));
-            x[s * 8 + 2 * j + 1] = bf16f((uint16_t)(w[j] >> 16));
-          }
+          for (int j = 0; j < 4; j++) x[s * 4 + j] = -INFINITY;
         }
       } else {
-#pragma unroll
-        for (int j = 0; j < VEC; j++) x[s * VEC + j] = -INFINITY;
+        r.v[s] = vu4{0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u};
+        if (i0 < hi) r.v[s] = *gmem((const vu4*)(base + (size_t)i0 * 2));
       }
     }
+  }
+  __device__ static inline void unpack(const Raw& r, float (&x)[EPT]) {
+    if constexpr (DT != QWS_DTYPE_F32) {
+#pragma unroll
+      for (int s = 0; s < S; s++) {
+        const uint32_t w[4] = {r.v[s].x, r.v[s].y, r.v[s].z, r.v[s].w};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          x[s * 8 + 2 * j] = bf16f((uint16_t)(w[j] & 0xFFFFu));
+          x[s * 8 + 2 * j + 1] = bf16f((uint16_t)(w[j] >> 16));
+        }
+      }
+    }
+  }
+  // Raw logits of block [lo, hi) of `row`, -inf past hi
+  __device__ static inline void load_raw(const qws_batch& B, int row, int lo, int hi, float (&x)[EPT]) {
+    Raw r;
+    load_bits(B, row, lo, hi, r, x);
+    unpack(r, x);
   }
   __device__ static inline void fixnan(float (&x)[EPT]) {
 #pragma unroll
@@ -195,7 +215,7 @@ __device__ inline float proc_one(float x, uint32_t t, const qws_row& R, const fl
 // other threads still read the table, which saves two barriers.  LB (listed processing; list2 then holds lcap2 words
 // and `bits` is BLK / 32 words of LDS): the touched tokens are listed by local index, from a bitmap the marks also
 // set (short histories) or from the table words, each is processed by one thread from its word and a second read of
-// its logit, and the values go back through the table (no compaction of the owners' values).  Under LB an fp32 row
+// its logit, and the values go back through the table (no compaction of the owners' values).  Under LB a row
 // whose only list is its state slot (distinct tokens with their counts) takes a shorter form: each entry is processed
 // in place in a table of the block's values.  tail = false leaves out the final barrier: the caller
 // then orders its next writes to tab (and list2, bits) after a barrier of its own.
@@ -206,14 +226,17 @@ __device__ inline void load_processed(const qws_batch& B, const qws_row& R, int 
   using BL = Blk<DT, NTH>;
   constexpr int EPT = BL::EPT;
   // every global load of the block is issued before the first wait: logits, mask words, the first list entries
-  BL::load_raw(B, row, lo, hi, x);
+  typename BL::Raw raw;
+  BL::load_bits(B, row, lo, hi, raw, x);
   if (!R.proc_on) {
+    BL::unpack(raw, x);
     BL::fixnan(x);
     return;
   }
   uint32_t mw[BL::S];
   BL::mask_words(B, R, lo, hi, mw);
   if (!row_touches(B, R)) {
+    BL::unpack(raw, x);
     BL::fixnan(x);
     BL::apply_mask(R, lo, hi, mw, x);
     return;
@@ -242,11 +265,12 @@ __device__ inline void load_processed(const qws_batch& B, const qws_row& R, int 
     if (tid < sn) se0 = gmem(sent)[tid];
   }
   uint4* t4 = (uint4*)tab;
-  if constexpr (LB && DT == QWS_DTYPE_F32) {  // (bf16 rows: their 64-register workgroups would spill in the loads)
+  if constexpr (LB) {
     if (sslot >= 0 && Ls.e == 0) {
       // State alone: its entries are distinct tokens with their counts, so nothing is marked.  The owners put the
       // block's values in the table (token order), each entry's thread processes its token there, and the owners
       // read the values back: two barriers, no listing, no second read of the logits.
+      BL::unpack(raw, x);
       BL::fixnan(x);
       BL::apply_mask(R, lo, hi, mw, x);
       if (sn == 0) {  // uniform: the slot touches nothing in this block
@@ -315,6 +339,7 @@ __device__ inline void load_processed(const qws_batch& B, const qws_row& R, int 
   // the logits arrived before the first list entries (loads complete in order): NaN and the mask now, so that the
   // mask words die here (a masked touched token still ends -inf: its processed value is read through `at`, or
   // computed in place from the -inf)
+  BL::unpack(raw, x);
   BL::fixnan(x);
   BL::apply_mask(R, lo, hi, mw, x);
   for (int j0 = PF * NTH; j0 < Ls.b; j0 += PF * NTH) {  // the rest of a long history, PF loads in flight per thread
