@@ -18,8 +18,16 @@ struct RowRes {
   float K;                        // kscale(T)
   int kind;                       // RR_*
   int tok;                        // the row's own draw from p (the greedy token for RR_GREEDY, 0 for RR_EMPTY)
-  int pad;
+  int n_kept;                     // > 0: the kept set is in the row's KeptSet (at most 64 tokens)
 };
+// The kept tokens of a row that one wave finished, in rank order with their weights (row units): the verify kernels draw
+// its residual from them, with no pass over its blocks.  One per row, after the call's RowRes array.
+struct KeptSet {
+  unsigned long long w[64];
+  unsigned idx[64];
+};
+__host__ __device__ inline size_t rowres_bytes(int B) { return ((size_t)B * sizeof(RowRes) + 255) & ~(size_t)255; }
+__host__ __device__ inline KeptSet* kept_sets(const RowRes* r, int B) { return (KeptSet*)((char*)r + rowres_bytes(B)); }
 enum : int { RR_FAIL = -1, RR_EMPTY = 0, RR_GREEDY = 1, RR_SAMPLED = 2 };
 
 // Extra work of k_scan / k_resolve for the rows of a verify call (all null / 0 for qws_sample).

@@ -1333,7 +1333,7 @@ __device__ __forceinline__ void advance_row(const qws_batch& B, const qws_row& R
 // returns the row's token (-1: none) once its outputs are written.  Out of line: inlined into k_resolve it slowed the
 // general rows by its place in the code (C4 resolve 20.5 -> 22.4 us).
 struct TopRow {
-  int row, V, G, K;
+  int row, V, G, K, B;
   uint32_t u_draw;
   float temperature, top_p, min_p;
   double log2_min_p;
@@ -1437,6 +1437,11 @@ __device__ __forceinline__ int finish_ranked(const TopRow& A, int n, const uint6
       const double S2d = (double)(uint64_t)(S2 >> 64) * 18446744073709551616.0 + (double)(uint64_t)S2;
       A.out_probs[(size_t)A.row * A.V + idx] = (float)((double)w / S2d);
     }
+    if (VER && lane < m) {
+      KeptSet& ks = kept_sets(A.rres, A.B)[A.row];
+      ks.w[lane] = w;
+      ks.idx[lane] = idx;
+    }
     const int rl = readlane<int>(r, max(m - 1, 0));
     const uint64_t cl = readlane<uint64_t>(cc, max(m - 1, 0));
     if (lane == 0) {
@@ -1453,6 +1458,7 @@ __device__ __forceinline__ int finish_ranked(const TopRow& A, int n, const uint6
           o.cR = rl;
           o.row_top = row_top;
           o.K = Ks;
+          o.n_kept = m;
         }
         A.rres[A.row] = o;
       }
@@ -1531,6 +1537,7 @@ __device__ __forceinline__ TopRow top_row(QWS_L const TopRow* a) {
   A.V = __builtin_amdgcn_readfirstlane(a->V);
   A.G = __builtin_amdgcn_readfirstlane(a->G);
   A.K = __builtin_amdgcn_readfirstlane(a->K);
+  A.B = __builtin_amdgcn_readfirstlane(a->B);
   A.u_draw = a->u_draw;
   A.temperature = a->temperature;
   A.top_p = a->top_p;
@@ -1721,7 +1728,7 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
   bar();
   __shared__ TopRow s_top;
   if (listed_top(R)) {  // uniform
-    if (tid == 0) s_top = TopRow{row, B.V, G, R.top_k, u_draw, R.temperature, R.top_p, R.min_p, R.log2_min_p, 0, 0, B.out_tokens, B.out_info, B.out_probs, rres};
+    if (tid == 0) s_top = TopRow{row, B.V, G, R.top_k, B.B, u_draw, R.temperature, R.top_p, R.min_p, R.log2_min_p, 0, 0, B.out_tokens, B.out_info, B.out_probs, rres};
     bar();
     const int tk = resolve_top<VER>((QWS_L const TopRow*)&s_top, (QWS_L const char*)s_fb, (QWS_L const float2*)S.ts, (QWS_L char*)S.big);
     if (!VER && B.advance) advance_row(B, R, row, tk, &S.nt, -1, 0, 0u);
@@ -1843,7 +1850,7 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
       const int e0 = __shfl(exc, min(g, 63));
       T.lst[lane] = lane < tot ? els_of(ws, G, row, g)[lane - e0] : 0ull;
       if (lane == 0)
-        s_top = TopRow{row, B.V, G, 64, u_draw, R.temperature, R.top_p, thr == 0 ? R.min_p : 0.0f, R.log2_min_p, (unsigned long long)thr,
+        s_top = TopRow{row, B.V, G, 64, B.B, u_draw, R.temperature, R.top_p, thr == 0 ? R.min_p : 0.0f, R.log2_min_p, (unsigned long long)thr,
                        (unsigned long long)(thr >> 64), B.out_tokens, B.out_info, B.out_probs, rres};
     } else if (wave_id() == 1) {
       T.lst[64 + lane] = 0ull;
@@ -2029,7 +2036,7 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
       o.K = K;
       o.kind = RR_SAMPLED;  // tok = -1: not drawn here
       o.tok = tok;
-      o.pad = 0;
+      o.n_kept = 0;
       rres[row] = o;
     }
   }

@@ -87,35 +87,49 @@ __device__ inline u128 q_fix(float q, u128 S2) {
 
 __device__ inline u128 s2_of(const RowRes& rr) { return rr.kind == RR_GREEDY ? (u128)1 : (((u128)rr.s_hi << 64) | rr.s_lo); }
 
-// The test of row t of sequence b: returns true when the row ends the sequence (t == K, a row without a sampled
-// distribution to test against, or a rejected draft); *rej = a draft was rejected against a sampled row, *flags = the
-// row's test flags.  ts: the exp2 table (LDS copy).
-__device__ inline bool verify_stop(const VerifyArgs& A, int b, int t, bool* rej, const float2* ts, int* flags) {
-  *rej = false;
+// What the test of row t of sequence b reads, every load issued together (t <= K)
+struct VTest {
+  RowRes rr;
+  unsigned long long seed;
+  unsigned position, stream, row_key;
+  int flags, d;
+  float x, q;
+};
+__device__ inline VTest verify_load(const VerifyArgs& A, int b, int t) {
+  VTest v;
   const int row = b * (A.K + 1) + t;
-  const qws_row R = A.T.rows[row];  // loaded with the row's result, before either is used
-  const RowRes rr = A.rres[row];
-  *flags = R.test_flags;
+  const qws_row& R = A.T.rows[row];
+  v.rr = A.rres[row];
+  v.seed = R.seed;
+  v.position = R.position;
+  v.stream = R.stream;
+  v.row_key = R.row_key;
+  v.flags = R.test_flags;
+  v.d = t < A.K ? A.dtok[b * A.K + t] : -1;
+  v.x = A.vx[row];  // written by the blocks holding the drafts: used for drafts inside the vocabulary only
+  v.q = A.vq[row];
+  return v;
+}
+// The test of row t: returns true when the row ends the sequence (t == K, a row without a sampled distribution to test
+// against, or a rejected draft); *rej = a draft was rejected against a sampled row.  ts: the exp2 table (LDS copy).
+__device__ inline bool verify_stop(const VerifyArgs& A, const VTest& v, int t, bool* rej, const float2* ts) {
+  *rej = false;
+  const RowRes& rr = v.rr;
   if (t >= A.K || rr.kind == RR_EMPTY || rr.kind == RR_FAIL) return true;
-  const int V = A.T.V;
-  const int d = A.dtok[b * A.K + t];
-  const bool dok = d >= 0 && d < V;
+  const bool dok = v.d >= 0 && v.d < A.T.V;
   const u128 S2 = s2_of(rr);
   uint64_t wd = 0;
   if (dok) {
     if (rr.kind == RR_GREEDY) {
-      wd = d == rr.tok ? 1u : 0u;
-    } else {
-      const float x = A.vx[row];
-      if (x != -INFINITY) {
-        const W w = weigh(tval(x, rr.K), ts);
-        const int r = rr.row_top - w.bin();
-        if (r < NBIN && (r < rr.cR || (r == rr.cR && comp(okey(x), (uint32_t)d) >= rr.cC))) wd = row_weight(w.mu, r);
-      }
+      wd = v.d == rr.tok ? 1u : 0u;
+    } else if (v.x != -INFINITY) {
+      const W w = weigh(tval(v.x, rr.K), ts);
+      const int r = rr.row_top - w.bin();
+      if (r < NBIN && (r < rr.cR || (r == rr.cR && comp(okey(v.x), (uint32_t)v.d) >= rr.cC))) wd = row_weight(w.mu, r);
     }
   }
-  const float qv = dok ? A.vq[row] : 0.0f;  // recorded by the block holding d
-  const uint32_t u = draw_u24(R.seed, R.position, R.stream, R.row_key, 0);
+  const float qv = dok ? v.q : 0.0f;
+  const uint32_t u = draw_u24(v.seed, v.position, v.stream, v.row_key, 0);
   if ((u128)u * q_fix(qv, S2) < ((u128)wd << 24)) return false;  // accept w.p. min(1, p / q)
   *rej = rr.kind == RR_SAMPLED;
   return true;
@@ -198,19 +212,27 @@ __global__ void __launch_bounds__(NT3) k_vres(VerifyArgs A) {
   using BL = Blk<DT, NT3>;
   __shared__ __attribute__((aligned(16))) uint32_t s_tab[BLK];
   __shared__ __attribute__((aligned(16))) float2 s_ts[1024];
-  __shared__ int s_nt, s_vs;
+  __shared__ int s_nt, s_vs, s_any;
   __shared__ u128 s_red[68];
   const int b = blockIdx.x / A.G, g = blockIdx.x - b * A.G, tid = threadIdx.x;
-  // the exp2 table first: the tests weigh from its LDS copy (no global table read after the rows' loads)
+  VTest vt = {};
+  if (tid <= A.K) vt = verify_load(A, b, tid);  // lanes of the first wave
+  // the exp2 table with them: the tests weigh from its LDS copy
   for (int i = tid; i < 512; i += NT3) ((uint4*)s_ts)[i] = ((const uint4*)EXP2_TS)[i];
+  if (tid < 64) {
+    // a sequence whose every row has its kept set listed (or needs none) needs no block: its block 0 alone tests
+    const bool block = tid <= A.K && vt.rr.kind == RR_SAMPLED && vt.rr.n_kept == 0;
+    const bool any = g == 0 || __ballot(block) != 0ull;
+    if (tid == 0) s_any = any ? 1 : 0;
+  }
   bar();
+  if (s_any == 0) return;  // uniform
   if (tid < 64) {  // lane t tests row t; the first row that ends the sequence is t* (lane K always stops)
     bool rej = false;
-    int fl = 0;
-    const bool stop = tid > A.K || verify_stop(A, b, tid, &rej, s_ts, &fl);
+    const bool stop = tid > A.K || verify_stop(A, vt, tid, &rej, s_ts);
     const int ts = first_lane(stop);
     const bool need = ballot_bit(rej, ts);
-    const int flags = readlane<int>(fl, ts);  // row t*'s test flags, loaded by lane t*
+    const int flags = readlane<int>(vt.flags, ts);  // row t*'s test flags, loaded by lane t*
     if (tid == 0) {
       s_vs = ts | ((need && !(flags & QWS_TF_BROKEN)) ? 256 : 0);
       if (g == 0) A.vs[b] = s_vs;
@@ -221,7 +243,7 @@ __global__ void __launch_bounds__(NT3) k_vres(VerifyArgs A) {
   const int t = vs & 255, row = b * (A.K + 1) + t;
   const RowRes rr = A.rres[row];
   const bool res = vs & 256, plain = rr.kind == RR_SAMPLED && rr.tok < 0;  // the row's draw from p not taken yet
-  if (!res && !plain) return;
+  if ((!res && !plain) || rr.n_kept > 0) return;  // uniform; a listed kept set: k_vfin draws the residual from it
   const qws_row R = A.T.rows[row];
   uint64_t wv[BL::EPT], kp;
   residual_block<DT, NT3>(A, R, rr, b, t, row, g, s_tab, &s_nt, s_ts, wv, res, &kp);
@@ -274,32 +296,92 @@ __global__ void __launch_bounds__(NT3) k_vfin(VerifyArgs A) {
   constexpr bool CH = NT3 == NT3L;             // chunk prefixes are recorded at NT3L only
   constexpr int NCH = CH ? BL::S * NWV3 : 1;  // chunks per block
   __shared__ u128 s_chp[CH ? MAXG * NCHMAX : 1];
-  const int b = blockIdx.x, tid = threadIdx.x;
+  const int b = blockIdx.x, tid = threadIdx.x, G = A.G;
   const int vs = A.vs[b];
   const int t = vs & 255, row = b * (A.K + 1) + t;
   const RowRes rr = A.rres[row];
   const qws_row R = A.T.rows[row];
+  // every block's chunk prefixes (k_vres at NT3L), loaded behind the row's result and before it is looked at
+  const bool chunked = CH && A.chunked;
+  constexpr int CPT = CH ? (MAXG * NCHMAX + NT3 - 1) / NT3 : 1;
+  vu4 cpv[CPT];
+  if (chunked) {
+    const unsigned long long* cp = A.chunkp + 2 * ((size_t)b * G * NCHMAX);
+#pragma unroll
+    for (int k = 0; k < CPT; k++) {
+      const int i = tid + k * NT3;
+      if (i < G * NCH) cpv[k] = gmem((const vu4*)(cp + 2 * ((size_t)(i / NCH) * NCHMAX + i % NCH)))[0];
+    }
+  }
+  if (rr.n_kept > 0) {  // uniform: the row's kept set is listed and its draw from p taken: only a residual is left to draw
+    int tok = rr.tok;
+    if (vs & 256) {
+      const int n = rr.n_kept, lane = lane_id(), w = wave_id();
+      const KeptSet& ks = kept_sets(A.rres, A.T.B)[row];
+      // every wave: the residual weights max(0, w - floor(q S2)), one kept token per lane (as residual_block)
+      const uint32_t idx = lane < n ? ks.idx[lane] : 0xFFFFFFFFu;
+      uint64_t wv = lane < n ? ks.w[lane] : 0ull;
+      float qv = 0.0f;
+      if (A.nchain && t >= A.nchain[b]) {
+        qv = lane < n && (int)idx == A.dtok[b * A.K + t] ? 1.0f : 0.0f;
+      } else if (lane < n) {
+        const int iv = A.inv[idx];
+        if (iv >= 0 && iv < A.Vd) qv = A.dprob[((size_t)b * A.K + t) * A.Vd + iv];
+      }
+      if (qv > 0.0f) {
+        const u128 qf = q_fix(qv, s2_of(rr));
+        wv = (u128)wv > qf ? wv - (uint64_t)qf : 0;
+      }
+      // the draw in index order: wave p sums, for each token, the weights of tokens p, p + NWV3, ... with a lower index
+      // (at most eight, below 2^62), wave 0 adds the sums up
+      static_assert(64 / NWV3 <= 8, "partial sums below 2^62");
+      uint64_t part = 0;
+#pragma unroll
+      for (int j = 0; j < 64 / NWV3; j++) {
+        const int i = __builtin_amdgcn_readfirstlane(w) + j * NWV3;
+        const uint32_t ij = readlane<uint32_t>(idx, i);
+        const uint64_t wj = readlane<uint64_t>(wv, i);
+        part += ij < idx ? wj : 0ull;
+      }
+      uint64_t* sp = (uint64_t*)s_tab;  // [NWV3][64]
+      sp[w * 64 + lane] = part;
+      bar();
+      if (w == 0) {
+        u128 below = 0;
+#pragma unroll
+        for (int p = 0; p < NWV3; p++) below += sp[p * 64 + lane];
+        const u128 Rt = wave_sum_u128((u128)wv);
+        if (Rt != 0) {  // uniform (zero: the draw from p)
+          const u128 tt = mul_shr_floor(Rt, draw_u24(R.seed, R.position, R.stream, R.row_key, R.draw_word), 24);
+          const int l = first_lane(wv != 0 && below <= tt && tt < below + wv);
+          if (l < 64) tok = (int)readlane<uint32_t>(idx, l);
+        }
+      }
+    }
+    if (tid == 0) s_tok = tok;
+    bar();
+    const int Kd = A.K;
+    for (int j = tid; j <= Kd; j += NT3) A.out_tokens[(size_t)b * (Kd + 1) + j] = j < t ? A.dtok[b * Kd + j] : (j == t ? s_tok : -1);
+    if (tid == 0) A.out_n[b] = t + 1;
+    return;
+  }
   if (tid == 0) {
     s_g = -1;
     s_tok = rr.tok;
     s_plain = 0;
   }
   // the blocks' masses (lane g: block g's) loaded together with the exp2 table
-  const int G = A.G;
   u128 kres = 0, kkept = 0;
   if (tid < G) {
     const unsigned long long* pw = A.part + 4 * ((size_t)b * G + tid);
     if (vs & 256) kres = ((u128)pw[1] << 64) | pw[0];
     if (rr.kind == RR_SAMPLED && rr.tok < 0) kkept = ((u128)pw[3] << 64) | pw[2];
   }
-  // every block's chunk prefixes (k_vres at NT3L), loaded with the masses and the table
-  const bool chunked = CH && A.chunked;
   if (chunked) {
-    const unsigned long long* cp = A.chunkp + 2 * ((size_t)b * G * NCHMAX);
-    for (int i = tid; i < G * NCH; i += NT3) {
-      const int g = i / NCH, c = i - g * NCH;
-      const vu4 q = gmem((const vu4*)(cp + 2 * ((size_t)g * NCHMAX + c)))[0];
-      s_chp[g * NCHMAX + c] = ((u128)(((unsigned long long)q.w << 32) | q.z) << 64) | (((unsigned long long)q.y << 32) | q.x);
+#pragma unroll
+    for (int k = 0; k < CPT; k++) {
+      const int i = tid + k * NT3;
+      if (i < G * NCH) s_chp[(i / NCH) * NCHMAX + i % NCH] = ((u128)(((unsigned long long)cpv[k].w << 32) | cpv[k].z) << 64) | (((unsigned long long)cpv[k].y << 32) | cpv[k].x);
     }
   }
   for (int i = tid; i < 512; i += NT3) ((uint4*)s_ts)[i] = ((const uint4*)EXP2_TS)[i];
@@ -499,7 +581,7 @@ static VLayout vlayout(int Bs, int K, int V) {
   VLayout L;
   L.rows = 0;
   L.rres = al256(rows_ws_bytes((int)Bt, V));
-  L.vx = L.rres + al256(Bt * sizeof(RowRes));
+  L.vx = L.rres + al256(rowres_bytes((int)Bt) + Bt * sizeof(KeptSet));
   L.vq = L.vx + al256(Bt * 4);
   L.rtok = L.vq + al256(Bt * 4);
   L.part = L.rtok + al256(Bt * 4);
