@@ -294,8 +294,8 @@ __device__ __forceinline__ void stage_store(const RL& L, const qws_row& R, int g
 
 // Block g of the row, processed, into L.big in token order (tokens past V read -inf).  With the block's patches
 // recorded by k_scan the raw logits get the mask and the patches (the patches load together with the logits);
-// otherwise the processors are rebuilt from the row's lists.  B and R are the workgroup's LDS copies.  All threads;
-// ends with a barrier.
+// otherwise the processors are rebuilt from the row's lists.  B and R are the workgroup's LDS copies.  All threads, after a
+// barrier that follows the last reads of L.big; ends with a barrier.
 template <int DT>
 __device__ __forceinline__ void stage_block_body(const RL& L, const qws_batch& B, const qws_row& R, char* ws, int row, int g) {
   using BL = Blk<DT, NT2>;
@@ -516,7 +516,9 @@ __device__ __forceinline__ void for_bin(ResolveLds& S, char* ws, int row, F fn) 
 }
 
 // The blocks of st.gfast rescanned for the elements of row bin rb, into the gathered list.  Out of line: the rare path's
-// registers would spill the resolver's other paths.  All threads.
+// registers would spill the resolver's other paths.  All threads; ends with a barrier that hands L.big over: a block
+// staged next clears it before a barrier of its own (load_processed), and a wave still testing this function's last
+// bitmaps would take masked and processed tokens' raw values into the list.
 template <int DT>
 __device__ __noinline__ void rescan_fast(QWS_L ResolveLds* s, char* ws_, int row_, int rb_) {
   using BL = Blk<DT, NT2>;
@@ -627,6 +629,7 @@ __device__ __noinline__ void rescan_fast(QWS_L ResolveLds* s, char* ws_, int row
     atomicMin(&st.gmin, mn);
     atomicMax(&st.gmax, mx);
   }
+  bar();  // the bitmaps in L.big are read no more
 }
 
 // Gathers row bin rb (its power's fine bins staged): each block's elements come from its list when its window held

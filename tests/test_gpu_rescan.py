@@ -41,6 +41,35 @@ def test_rescans(sampler, blocks, dtype):
         check_rows(sampler, x, specs, label=f"blocks={blocks} flags={flags}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("slow", [(1,), (0, 7, 11)])
+def test_rescans_with_bitmaps_before_staged_blocks(sampler, slow, dtype):
+    """One row's cut bin rescanned both from blocks with masked and processed tokens (bitmaps) and from blocks with more
+    processed tokens than patches (staged afterwards in the bitmaps' LDS): every block holds 60 tokens of the bin, half of
+    them banned or penalised out of it, which must not come back with their raw values."""
+    blocks, V, n = 12, 12 * BLK, 60
+    params = [dict(top_p=0.5), dict(top_p=0.9), dict(top_k=150), dict(top_k=300, top_p=0.8), dict(min_p=0.998), dict(top_p=0.3, min_p=0.5)]
+    g = torch.Generator().manual_seed(len(slow))
+    x = torch.randn(2 * len(params), V, generator=g) - 9.0
+    rows = []
+    for b in range(2 * len(params)):
+        hot = torch.stack([k * BLK + torch.randperm(BLK, generator=g)[:n] for k in range(blocks)])  # per block: 15 banned, 15 penalised, 30 kept
+        x[b, hot.flatten()] = 5.0 + 0.004 * torch.rand(blocks * n, generator=g)  # a bin is 0.0108 wide at T = 1
+        out, gen = hot[:, :15].flatten(), hot[:, 15:30].flatten().tolist()
+        for k in slow:
+            cold = torch.ones(BLK, dtype=torch.bool)
+            cold[hot[k] - k * BLK] = False
+            gen += (k * BLK + torch.nonzero(cold).flatten()[:1025]).tolist()
+        touched = np.bincount(np.asarray(gen) // BLK, minlength=blocks)
+        assert all((touched[k] > 1024) == (k in slow) for k in range(blocks))
+        mask = np.zeros((V + 31) // 32, np.uint32)
+        np.bitwise_or.at(mask, out.numpy() >> 5, np.uint32(1) << (out.numpy() & 31).astype(np.uint32))
+        masks = dict(banned=mask) if b % 2 else dict(allowed=[i for i in range(V) if not (int(mask[i >> 5]) >> (i & 31)) & 1])
+        rows.append(q.RowSpec(temperature=1.0, repetition=1.2, presence=0.4, gen=gen, seed=b, position=b, row_key=b, test_flags=q.TF_RESCAN, **masks, **params[b // 2]))
+    info = check_rows(sampler, x.to(dtype), rows, label=f"slow={slow}")
+    assert info.tolist() == [1] * len(rows)  # every row's cut lies in the rescanned bin
+
+
 def test_min_p_below_a_top_k_cut(sampler):
     """A min-p cut far below the top-k cut is not looked up: no rescans (out_info 0), the same tokens; at and around the count
     above the min-p cut's bin both cuts still apply."""
