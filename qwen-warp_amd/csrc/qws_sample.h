@@ -1357,6 +1357,7 @@ struct TopBuf {
   uint64_t part[NWV2][64];                 // partial sums of the kept weights before a candidate in index order
   uint64_t bound;
   int cnt, tok;
+  int cnt2;                                // entries of the reduced list (its own word: late waves may still read cnt)
 };
 static_assert(TOP_NL1 <= NT2 / 4 && TOP_NL1 <= 64 * TOP_EPL && sizeof(TopBuf) <= BIGW * 4, "LDS of resolve_top");
 // Inclusive prefix over lanes of row weights (< 2^59 each: a row of 16 lanes sums to less than 2^63)
@@ -1525,10 +1526,10 @@ __device__ __forceinline__ int resolve_top_body(const TopRow& A, const char* hdr
         base += __popcll(bal);
       }
       for (int i = base + lane; i < TOP_NL1; i += 64) L.mxs[i] = 0ull;
-      if (lane == 0) L.cnt = base;
+      if (lane == 0) L.cnt2 = base;
     }
     bar();
-    n = __builtin_amdgcn_readfirstlane(L.cnt);
+    n = __builtin_amdgcn_readfirstlane(L.cnt2);
     src = L.mxs;
   }
   return finish_ranked<VER>(A, n, src, ts, L);

@@ -46,6 +46,26 @@ def test_top_list_rows(sampler, kind, V):
         check_rows(sampler, x.to(dt), rows, label=f"{kind} V={V} {dt}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("blocks,crowd", [(17, 3), (31, 3), (32, 3), (33, 6), (64, 7)])
+def test_top_list_rows_crowded_blocks(sampler, blocks, crowd, dtype):
+    """The best tokens crowded into a few blocks whose lists are held by fewer threads than top_k (16 threads per block up to
+    32 blocks, 8 past them): the resolver's bound falls below all of them, more than 128 entries reach it, and they are
+    reduced before they are ranked."""
+    V, tpb = blocks * 8192, 16 if blocks <= 32 else 8
+    assert crowd * tpb < 64 and crowd * 64 > 128
+    g = torch.Generator().manual_seed(blocks)
+    B = 10
+    x = torch.randn(B, V, generator=g) * 2.0
+    rows = []
+    for b in range(B):
+        for k in torch.randperm(blocks, generator=g)[:crowd].tolist():
+            x[b, k * 8192 + torch.randperm(8192, generator=g)[:300]] += 30.0
+        rows.append(q.RowSpec(temperature=[1.0, 8.0][b % 2], top_k=[64, 58, 64, 64, 60][b % 5], top_p=[1.0, 0.9][b // 2 % 2], seed=b, position=b, row_key=b))
+        assert rows[-1].top_k > crowd * tpb
+    check_rows(sampler, x.to(dtype), rows, label=f"blocks={blocks}")
+
+
 @pytest.mark.parametrize("B", [7, 40])
 def test_top_list_rows_with_processors(sampler, B):
     """Both k_scan widths (7 x 31 and 40 x 31 workgroups) with penalties, biases past the bound and masked tokens; rows
