@@ -341,8 +341,9 @@ class PackedBatch:
                 elif r.banned is not None:
                     mask_mode, mask_row = MASK_BANNED, len(masks)
                     masks.append(np.asarray(r.banned, dtype=np.uint32)[:W])
-                if mask_mode and masks[mask_row].shape != (W,):
-                    raise ValidationError(f"a mask must hold {W} words", "banned")
+                # W words in any shape (a row or a column of a bitmask matrix), the same one on every row of the batch
+                if mask_mode and (masks[mask_row].size != W or masks[mask_row].shape != masks[0].shape):
+                    raise ValidationError(f"a mask must hold {W} words, in one shape over the batch", "banned")
             vals = (r.temperature, r.top_k, r.top_p, r.min_p, math.log2(float(np.float32(r.min_p))) if r.min_p > 0 else 0.0, int(r.seed) & (2 ** 64 - 1),
                     r.position & 0xFFFFFFFF, r.stream, r.row_key & 0xFFFFFFFF, int(on), r.presence, r.frequency, r.repetition, r.min_tokens, ng, *lists, n_stop,
                     mask_mode, mask_row, r.test_flags, r.draw_word, st if st >= 0 else -1, 0)
@@ -368,9 +369,9 @@ class PackedBatch:
         buf[:len(rowb)] = np.frombuffer(rowb, np.uint8)
         for o, arrs in zip(offs[1:], (hist, drafts, bids, None, stops, masks)):
             for a in arrs or ():
-                if len(a):
-                    buf[o:o + 4 * len(a)].view(np.uint32 if arrs is masks else np.int32)[:] = a
-                    o += 4 * len(a)
+                if a.size:
+                    buf[o:o + 4 * a.size].view(np.uint32 if arrs is masks else np.int32)[:] = a.reshape(-1)
+                    o += 4 * a.size
         if nb_all:
             buf[offs[4]:offs[4] + 4 * nb_all].view(np.float32)[:] = bvals
         self.dev_buf = host.to(dev, non_blocking=ordered)

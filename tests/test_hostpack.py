@@ -50,6 +50,19 @@ def test_packed_rows_fields():
         q.PackedBatch([q.RowSpec(banned=np.zeros(3, np.uint32))], V, "cpu")
 
 
+@pytest.mark.parametrize("shape", [(1, -1), (-1, 1), (4, -1), (2, -1, 1)])
+def test_masks_of_other_shapes(shape):
+    """A banned mask of the right number of words is taken in any shape, the same one on every masked row."""
+    words = np.random.default_rng(1).integers(0, 1 << 32, 32, dtype=np.uint32)
+    flat = q.PackedBatch([q.RowSpec(banned=words), q.RowSpec(), q.RowSpec(banned=~words)], V, "cpu")
+    p = q.PackedBatch([q.RowSpec(banned=words.reshape(shape)), q.RowSpec(), q.RowSpec(banned=~words.reshape(shape))], V, "cpu")
+    assert torch.equal(p.masks_t, flat.masks_t) and torch.equal(p.dev_buf, flat.dev_buf)
+    assert np.array_equal(p.masks_t.numpy().view(np.uint32), np.stack([words, ~words]))
+    for rows in ([q.RowSpec(banned=words.reshape(shape)), q.RowSpec(banned=words)], [q.RowSpec(banned=words[:31])], [q.RowSpec(banned=words), q.RowSpec(banned=words[None, :31])]):
+        with pytest.raises(ValueError):
+            q.PackedBatch(rows, V, "cpu")
+
+
 @pytest.mark.gpu
 def test_ordered_copies_back_to_back(sampler):
     """Calls that pack their own rows, issued without waiting: each runs on its own rows (staging buffers are not reused early)."""
