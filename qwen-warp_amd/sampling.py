@@ -221,12 +221,14 @@ _NO_IDS.flags.writeable = False
 def _ids(ids, V, name) -> np.ndarray:
     """Token ids (a list, tuple, set, dict keys, numpy array or tensor) as one int64 array in iteration order, converted
     once; ValidationError unless every id is an integer in [0, V) (a float or bool array is refused, not truncated)."""
-    if type(ids) is list or type(ids) is tuple:  # exact ints in range: one native pass
+    if type(ids) is list or type(ids) is tuple:
         if not ids:
             return _NO_IDS
-        a = np.empty(len(ids), np.int64)
-        if _lib.hostpack().ids(ids, V, a) == len(ids):
-            return a
+        native = _lib.hostpack()
+        if native is not None:  # exact ints in range: one native pass
+            a = np.empty(len(ids), np.int64)
+            if native.ids(ids, V, a) == len(ids):
+                return a
     if isinstance(ids, torch.Tensor):
         if ids.numel() and (ids.dtype == torch.bool or ids.dtype.is_floating_point or ids.dtype.is_complex):  # empty: any dtype
             raise ValidationError(f"{name}: token ids must be integers, got a {ids.dtype} tensor", name)

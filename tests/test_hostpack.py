@@ -29,6 +29,24 @@ def test_ids_refusals(bad):
             _ids(ids, V, "gen")
 
 
+@pytest.mark.parametrize("file", [None, b"not an extension"])
+def test_without_the_native_module(file, tmp_path, monkeypatch):
+    """A checkout without the module, or with one this interpreter cannot load: the general path, with the same rows and refusals."""
+    rows = [q.RowSpec(gen=[1, 2, 2], drafts=(3,), bias={4: 0.5}, stop=[6], min_tokens=9, allowed=[1, 33], repetition=1.1), q.RowSpec(prompt=[V - 1], presence=1.0)]
+    want = q.PackedBatch(rows, V, "cpu").dev_buf
+    path = tmp_path / _lib.HOSTPACK_PATH.name
+    if file:
+        path.write_bytes(file)
+    monkeypatch.setattr(_lib, "HOSTPACK_PATH", path)
+    monkeypatch.setattr(_lib, "_HOSTPACK", None)
+    with pytest.warns(RuntimeWarning, match="packed in Python"):
+        assert _lib.hostpack() is None
+    assert torch.equal(q.PackedBatch(rows, V, "cpu").dev_buf, want) and _ids([], V, "gen").size == 0
+    for bad in (-1, V, 2 ** 70, True, 1.0, "1"):
+        with pytest.raises(q.ValidationError):
+            _ids([1, bad], V, "gen")
+
+
 def test_ids_buffer_too_small():
     assert _lib.hostpack().ids([1, 2, 3], V, np.empty(2, np.int64)) == -1
 
