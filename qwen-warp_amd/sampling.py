@@ -268,6 +268,14 @@ _BATCH = struct.Struct("@P 3i q 7P i 4P P 2i")             # include/qws.h qws_b
 assert _ROW.size == C.sizeof(Row) and _BATCH.size == C.sizeof(Batch)
 
 
+def _capture_mode(mode: int) -> int:
+    """Sets the calling thread's stream capture mode (hipStreamCaptureMode: 0 global, 1 thread-local, 2 relaxed), returns the
+    mode before."""
+    m = C.c_int(mode)
+    check(_lib.load().hipThreadExchangeStreamCaptureMode(C.byref(m)), "hipThreadExchangeStreamCaptureMode")
+    return m.value
+
+
 class PackedBatch:
     """Rows packed into device arrays (CSR histories, bias, stop ids, masks) and the qws_batch struct.  Rows with a
     state_slot take their prompt set and generated counts from `state` (a ProcState) instead of a CSR history:
@@ -366,17 +374,25 @@ class PackedBatch:
             offs.append(n)
             n += (z + 255) & ~255
         ordered = ordered and dev.type == "cuda" and not torch.cuda.is_current_stream_capturing()
-        host = torch.empty(n, dtype=torch.uint8, pin_memory=True) if ordered else torch.zeros(n, dtype=torch.uint8)
-        buf = host.numpy()
-        buf[:len(rowb)] = np.frombuffer(rowb, np.uint8)
-        for o, arrs in zip(offs[1:], (hist, drafts, bids, None, stops, masks)):
-            for a in arrs or ():
-                if a.size:
-                    buf[o:o + 4 * a.size].view(np.uint32 if arrs is masks else np.int32)[:] = a.reshape(-1)
-                    o += 4 * a.size
-        if nb_all:
-            buf[offs[4]:offs[4] + 4 * nb_all].view(np.float32)[:] = bvals
-        self.dev_buf = host.to(dev, non_blocking=ordered)
+        # the pinned buffer's allocation and its events are allowed while another thread captures a graph: they touch no
+        # capturing stream, but in the default (global) mode they would fail and end that capture
+        mode = _capture_mode(2) if ordered else 0
+        try:
+            host = torch.empty(n, dtype=torch.uint8, pin_memory=True) if ordered else torch.zeros(n, dtype=torch.uint8)
+            buf = host.numpy()
+            buf[:len(rowb)] = np.frombuffer(rowb, np.uint8)
+            for o, arrs in zip(offs[1:], (hist, drafts, bids, None, stops, masks)):
+                for a in arrs or ():
+                    if a.size:
+                        buf[o:o + 4 * a.size].view(np.uint32 if arrs is masks else np.int32)[:] = a.reshape(-1)
+                        o += 4 * a.size
+            if nb_all:
+                buf[offs[4]:offs[4] + 4 * nb_all].view(np.float32)[:] = bvals
+            self.dev_buf = host.to(dev, non_blocking=ordered)
+            del host, buf
+        finally:
+            if ordered:
+                _capture_mode(mode)
         view = [self.dev_buf[o:o + z] for o, z in zip(offs, sizes)]
         self.rows_t = view[0]
         self.hist_t, self.drafts_t, self.bids_t = view[1].view(torch.int32), view[2].view(torch.int32), view[3].view(torch.int32)

@@ -1,4 +1,6 @@
 """The native id-list pass and the packed rows: the same arrays and refusals as the general Python path."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -92,3 +94,45 @@ def test_ordered_copies_back_to_back(sampler):
     want = [sampler.run(q.PackedBatch(rows, Vg, "cuda"), x).tolist() for rows in batches]
     got = [sampler.sample(x, rows) for rows in batches]
     assert [t.tolist() for t in got] == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("own_stream", [False, True])
+def test_packing_while_another_thread_captures(sampler, own_stream):
+    """Calls that pack their own rows, on one thread, while another captures a graph of the same library: both go on."""
+    Vg = 8 * 4096
+    x = torch.randn(4, Vg, generator=torch.Generator().manual_seed(1)).cuda()
+    rows = [q.RowSpec(temperature=1.0, top_p=0.9, seed=i, row_key=i) for i in range(4)]
+    other = [[q.RowSpec(temperature=1.0, top_p=0.9, repetition=1.2, gen=list(range(n + own_stream)), seed=i, row_key=i) for i in range(4)]
+             for n in (100, 3000, 20000, 3000)]  # staging buffers of several sizes: taken anew, and again
+    packed, out = q.PackedBatch(rows, Vg, "cuda"), torch.empty(4, dtype=torch.int32, device="cuda")
+    want, graph_sampler = sampler.run(packed, x).tolist(), q.Sampler("cuda")
+    stream, side, graph = torch.cuda.Stream() if own_stream else torch.cuda.current_stream(), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    capturing, packed_all, got = threading.Event(), threading.Event(), []
+
+    def serve():
+        try:
+            capturing.wait(30)
+            with torch.cuda.stream(stream):
+                got.extend(sampler.sample(x, r) for r in other)
+        except Exception as e:
+            got.append(e)
+        packed_all.set()
+
+    t = threading.Thread(target=serve)
+    t.start()
+    with torch.cuda.stream(side):
+        graph_sampler.run(packed, x, out_tokens=out)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            capturing.set()
+            packed_all.wait(30)
+            graph_sampler.run(packed, x, out_tokens=out)
+    t.join(30)
+    torch.cuda.synchronize()
+    assert [g.tolist() for g in got] == [sampler.run(q.PackedBatch(r, Vg, "cuda"), x).tolist() for r in other]
+    for _ in range(3):
+        out.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert out.tolist() == want
