@@ -276,6 +276,12 @@ def _capture_mode(mode: int) -> int:
     return m.value
 
 
+def _may_order(dev: torch.device) -> bool:
+    """A copy to dev may be left unwaited: its stream is not captured (a captured copy would read the staging buffer again
+    at each replay).  The capture state is known for the current device's stream; another device's copy is waited for."""
+    return dev.type == "cuda" and dev.index in (None, torch.cuda.current_device()) and not torch.cuda.is_current_stream_capturing()
+
+
 class PackedBatch:
     """Rows packed into device arrays (CSR histories, bias, stop ids, masks) and the qws_batch struct.  Rows with a
     state_slot take their prompt set and generated counts from `state` (a ProcState) instead of a CSR history:
@@ -373,7 +379,7 @@ class PackedBatch:
         for z in sizes:
             offs.append(n)
             n += (z + 255) & ~255
-        ordered = ordered and dev.type == "cuda" and not torch.cuda.is_current_stream_capturing()
+        ordered = ordered and _may_order(dev)
         # the pinned buffer's allocation and its events are allowed while another thread captures a graph: they touch no
         # capturing stream, but in the default (global) mode they would fail and end that capture
         mode = _capture_mode(2) if ordered else 0

@@ -7,6 +7,7 @@ import torch
 
 import qwen_warp_amd as q
 from qwen_warp_amd import _lib
+from qwen_warp_amd import sampling as _sampling
 from qwen_warp_amd.sampling import _ids
 
 V = 1000
@@ -81,6 +82,20 @@ def test_masks_of_other_shapes(shape):
     for rows in ([q.RowSpec(banned=words.reshape(shape)), q.RowSpec(banned=words)], [q.RowSpec(banned=words[:31])], [q.RowSpec(banned=words), q.RowSpec(banned=words[None, :31])]):
         with pytest.raises(ValueError):
             q.PackedBatch(rows, V, "cpu")
+
+
+@pytest.mark.parametrize("dev,capturing,want", [("cpu", False, False), ("cuda", False, True), ("cuda:0", False, True), ("cuda:1", False, False),
+                                                ("cuda", True, False), ("cuda:0", True, False), ("cuda:1", True, False)])
+def test_copies_left_unwaited(dev, capturing, want, monkeypatch):
+    """Only to the current device (0 here), whose stream's capture state is the one that is asked for, and not under capture."""
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    copied = []
+    monkeypatch.setattr(torch, "empty", lambda n, dtype, pin_memory: copied.append(True) or torch.zeros(n, dtype=dtype))
+    monkeypatch.setattr(torch.Tensor, "to", lambda t, d, non_blocking=False: copied.append(non_blocking) or t)
+    monkeypatch.setattr(_sampling, "_capture_mode", lambda mode: 0)
+    q.PackedBatch([q.RowSpec()], V, dev, ordered=True)
+    assert copied == [True, True] if want else copied == [False]
 
 
 @pytest.mark.gpu
