@@ -32,15 +32,14 @@ constexpr int MARGIN_FLAT = 6, MARGIN_NEAR = 31;
 constexpr int CTOP = 256;
 constexpr int MAXG = 64;                     // blocks per row (V <= 524,288)
 constexpr int NR = NBIN;                     // row bins with a nonzero weight (row-relative, 0 = the top)
-constexpr int XN = 4096;                     // elements of one bin k_resolve holds in LDS
 constexpr unsigned long long M40 = (1ull << 40) - 1;
 
 // ---------------------------------------------------------------------------------------------- block record
-enum : int { RF_CAND = 1, RF_SAMP = 2, RF_TOP = 4 };  // RF_TOP: a top-list record (listed_top)
+enum : int { RF_CAND = 1, RF_SAMP = 2 };  // has a candidate; has bins (top-list records write no flags: listed_top)
 // Bins of a block are top-down: rel = (c * 64 + 63) - fine bin, so rel 0..63 is the power of two 2^c of the block's
 // best and rel >> 6 = e counts powers of two below it.  Elements with rel >= NBIN weigh nothing in any row.
 struct Rec {
-  uint32_t max_key, max_idx;     // best candidate (okey, lowest index); KEY_NEGINF: none
+  uint32_t max_key, max_idx;     // best candidate's okey (KEY_NEGINF: none); its lowest index on greedy rows, 0 on sampled ones
   int c, flags;                  // power of two of the best; RF_*
   int nbw;                       // bins written: rel 0 .. nbw - 1 (every bin a cut of any row can fall in)
   int w0, w1;                    // listed bins: rel in [w0, w1] (none when w0 > w1)
@@ -130,8 +129,8 @@ static_assert(MAXG * HDR_BYTES <= (size_t)MAXG * FB * 8, "the headers are staged
 static_assert(BLK / NT2 == 16, "a thread's 16 staged tokens start at word 17 t");
 
 struct BI {                      // a block as the resolver uses it
-  uint32_t max_key, max_idx;
-  int c, flags, nbw, n_patch;
+  uint32_t max_key;
+  int c, nbw, n_patch;
   int dn;                        // N - c (row powers of two above the block's top one); -1: nothing of it weighs in the row
   int gcnt, goff, gsrc, gofs;    // the bin being gathered: the block's count, list offset, source (0 none, 1 list, 2 rescan),
                                  // first slot in the gathered list
@@ -1745,9 +1744,7 @@ __global__ void __launch_bounds__(NT2) k_resolve(qws_batch B, int G, char* ws, R
       const Rec& H = hdr(tid);
       BI b;
       b.max_key = H.max_key;
-      b.max_idx = H.max_idx;
       b.c = H.c;
-      b.flags = H.flags;
       b.nbw = H.nbw;
       b.n_patch = (H.flags & RF_CAND) ? H.n_patch : -1;
       b.dn = -1;

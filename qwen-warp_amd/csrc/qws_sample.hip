@@ -114,11 +114,7 @@ __device__ __forceinline__ void list_top(const float (&x)[Blk<DT, NT1>::EPT], in
     }
     n = base;
   }
-  if (tid == 0) {  // a lane of the wave that cut the list
-    Rec* H = (Rec*)rec;
-    H->flags = n > 0 ? RF_CAND | RF_TOP : RF_TOP;
-    H->n_list = n;
-  }
+  if (tid == 0) ((Rec*)rec)->n_list = n;  // a lane of the wave that cut the list
 }
 
 // ---------------------------------------------------------------------------------------------- k_scan
@@ -150,7 +146,7 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
   int& s_nt = *(int*)(s_lds + O_SMALL + 68);
   int& s_relmin = *(int*)(s_lds + O_SMALL + 72);
   int& s_nl = *(int*)(s_lds + O_SMALL + 76);
-  int* const s_win = (int*)(s_lds + O_SMALL + 80);  // 8 words
+  int* const s_win = (int*)(s_lds + O_SMALL + 80);  // 5 words
   float* const s_redb = (float*)(s_lds + O_SMALL + 128);  // NWV1 <= 16: wave maxima of the biased tokens' values
   static_assert(NWV1 <= 16, "wave maxima");
 
@@ -504,14 +500,14 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
     if (lane == 0) {
       s_win[0] = w0;
       s_win[1] = w1;
-      s_win[4] = (int)n_list;
-      s_win[5] = min(r1, hard) + 1;
-      s_win[6] = (int)before;
+      s_win[2] = (int)n_list;
+      s_win[3] = min(r1, hard) + 1;
+      s_win[4] = (int)before;
       s_nl = 0;
     }
   }
   bar();
-  const int w0 = s_win[0], w1 = s_win[1], nbw = s_win[5];
+  const int w0 = s_win[0], w1 = s_win[1], nbw = s_win[3];
   // ---- the record: header, per-power sums, bin words (with the list slots of the listed bins)
   if (tid == 0) {
     H->max_key = okey(M);
@@ -521,7 +517,7 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
     H->nbw = nbw;
     H->w0 = w0;
     H->w1 = w1;
-    H->n_list = s_win[4];
+    H->n_list = s_win[2];
     H->n_patch = n_patch;
   }
   if (tid < NEXP) {
@@ -532,7 +528,7 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
   // a wave writes one power's bin words at a time; a listed bin's slot in the list = the candidates above it from w0 on
   // (the powers' prefix and one scan inside the power: no wave waits for another's)
   unsigned long long* BW = (unsigned long long*)(rec + BIN_OFF);
-  const uint32_t epc = lane < NEXP ? s_ecnt[lane] : 0u, eex = wave_scan_incl<uint32_t>(epc) - epc - (uint32_t)s_win[6];
+  const uint32_t epc = lane < NEXP ? s_ecnt[lane] : 0u, eex = wave_scan_incl<uint32_t>(epc) - epc - (uint32_t)s_win[4];
   for (int p = wave; p * FB < nbw; p += NWV1) {  // uniform in the wave
     const int r = p * FB + lane;
     const unsigned long long h = hist[r];
