@@ -426,8 +426,17 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
         n_list = nf;
       } else {
         int b = floor_r;
-        bool flat = false;
-        if (topp) {
+        uint32_t nb = nf;                // candidates down to b
+        bool top = false, flat = false;  // listed from the block's top; around a flat block's boundary
+        if (minp) {
+          // The row's min-p cut lies above the block's floor by what the row's best lies above the block's, about what the
+          // block's best lies above its G-th (the block is one of G).  Where at most the list's capacity lies above the cut
+          // expected so, the top is listed, else (below) the bins just above the floor.
+          uint32_t through;
+          const int d = cross_cnt((uint32_t)G, &through) - r0;  // G <= MAXG < nf: the crossing exists
+          top = cnt_to(max(floor_r - d, 0)) <= (uint32_t)CAP;
+        }
+        if (topp && !top) {
           // the block's own top-p boundary bp (mass crossing) and the power of its (CTOP + 1)-th candidate, both from
           // the power-level prefixes above and one fine-bin scan each (independent: issued together)
           const float mf = at_last ? readlane<float>(ims, NEXP - 1) : mass_to(floor_r);
@@ -478,13 +487,21 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
             }
           } else {
             b = min(floor_r, bp + MARGIN_NEAR);
+            if (b < floor_r) nb = cnt_to(b);
+            if (nb > (uint32_t)CAP) {  // uniform: at most a quarter of the list below bp, one lane per bin
+              static_assert(MARGIN_NEAR <= 64, "one lane per bin");
+              const bool in = bp + 1 + lane <= b;
+              const uint32_t pre = wave_scan_incl<uint32_t>(in ? (uint32_t)(hist[bp + 1 + lane] >> 40) : 0u);
+              nb = cnt_to(bp);
+              const int k = __popcll(__ballot(in && pre <= (uint32_t)CAP / 4u));
+              b = bp + k;
+              if (k > 0) nb += readlane<uint32_t>(pre, k - 1);
+            }
           }
         }
         if (!flat) {  // uniform
-          // one range of as many bins as the list holds: from the top when that reaches b (or a min-p floor, which lies
-          // higher in the row than in most of its blocks), else the bins ending at b
-          const uint32_t nb = b == floor_r ? nf : cnt_to(b);
-          if (minp || nb <= (uint32_t)CAP) {
+          // one range of as many bins as the list holds: from the top when that reaches b, else the bins ending at b
+          if (top || nb <= (uint32_t)CAP) {
             uint32_t through;
             w0 = 0;
             w1 = min(cross_cnt((uint32_t)CAP + 1u, &through) - 1, floor_r);  // nf > CAP: the crossing lies at or above floor_r
