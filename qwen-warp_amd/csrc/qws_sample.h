@@ -149,8 +149,9 @@ struct RS {                      // row state (LDS)
   int fpow;                      // row power of two whose fine bins are staged (-1: none)
   int gbin, gn, gl, gstaged;     // the gathered bin: row bin, elements, listed ones, held in LDS
   int gres;                      // blocks of the gathered bin rescanned (their window missed it)
-  unsigned long long gfast;      // bit g: block g is rescanned straight from its raw logits and patches
+  unsigned long long gfast;      // bit g: block g is rescanned from its raw logits and patches (rescan_fast)
   unsigned long long gslow;      // bit g: block g is rescanned through the staged block (more processed tokens than patches)
+  float xlo, xhi;                // the gathered bin's value interval (bin_edges), when gfast is not 0
   int rescans;                   // blocks rescanned because their window missed a bin
   float K;
   unsigned long long best;
@@ -468,20 +469,11 @@ __device__ inline int gblock_at(const RL& L, int G, int i) {
 }
 __device__ inline uint32_t mu_of_comp(uint64_t c, float K, const float2* ts) { return weigh(tval(okey_val(comp_key(c)), K), ts).mu; }
 
-// A value range that holds every x of row bin `qb` (floor(tval(x, K)) >> 4 == qb), for rescans that test the exact bin
-// only for values inside it.  t = fl(x * K) in [16 qb, 16 qb + 16) puts the exact product x * K within half an ulp of
-// that interval: within 1 below |t| < 2^24 and within 2^-24 |t| above, both inside the margins of 1 + 10^-5 |t| in t
-// (the float rounding of the edges divided by K is smaller still).  A bin at the clamps of t (x * K at or beyond
-// +-2^30) passes every value.
-struct XRange {
-  float lo, hi;
-  __device__ inline bool maybe(float v) const { return v >= lo && v <= hi; }
-};
-__device__ inline XRange bin_xrange(int qb, float K) {
-  const long long t0 = 16ll * qb;
-  if (!(t0 > -(1ll << 30) + 16 && t0 + 32 < (1ll << 30))) return {-INFINITY, INFINITY};
-  const double lo = (double)(t0 - 1) - fabs((double)t0) * 1e-5, hi = (double)(t0 + 17) + fabs((double)(t0 + 16)) * 1e-5;
-  return {(float)(lo / (double)K), (float)(hi / (double)K)};
+// The values x of the bin with floor(tval(x, K)) >> 4 == qb: xlo <= x < xhi exactly (tval is monotone in x; NaN and -inf lie
+// outside).  False where the edges are no exact floats or lie at the clamps of t, or first_x_t gives up.
+__device__ inline bool bin_edges(int qb, float K, float* xlo, float* xhi) {
+  if (qb <= -(1 << 19) || qb >= (1 << 19)) return false;  // |t| < 2^23 + 16: multiples of 16 are exact
+  return first_x_t((float)(16 * qb), K, xlo) && first_x_t((float)(16 * qb + 16), K, xhi) && *xlo > -INFINITY;
 }
 
 // Calls fn(comp, mu) for every candidate of row bin rb (gathered: from LDS; else from the blocks' lists and rescans).
@@ -520,10 +512,18 @@ __device__ __forceinline__ void for_bin(ResolveLds& S, char* ws, int row, F fn) 
   bar();
 }
 
-// The blocks of st.gfast rescanned for the elements of row bin rb, into the gathered list.  Out of line: the rare path's
-// registers would spill the resolver's other paths.  All threads; ends with a barrier that hands L.big over: a block
-// staged next clears it before a barrier of its own (load_processed), and a wave still testing this function's last
-// bitmaps would take masked and processed tokens' raw values into the list.
+// The blocks of st.gfast rescanned for the elements of row bin rb, into the gathered list: their raw logits, streamed through
+// registers RD blocks deep, each value tested against the bin's interval (bin_edges).  A wave counts its hits in a block,
+// takes their slots with one atomic and writes their comps; the mantissas follow for all of them at the end, one per
+// thread.  Masked and processed tokens are marked in a bitmap per block (in L.big) that takes raw values out, and the
+// patches' values are tested themselves.  (Through the staged block, one at a time, a block costs ~5 us.)
+// Bound by what one CU loads (~16 bytes per cycle: 31 fp32 blocks 26 us) and the tests beside it.  Out of line: the rare
+// path's registers would spill the resolver's other paths; few of them and little code (15 KB), since it saves its callers'
+// and every call fetches it anew.  32 rows, k_resolve: one block missed 29.0 -> 26.1 us, 31 missed 68.8 -> 59.1, 31 missed for
+// each of two cuts 171.7 -> 112.7, against batches of eight blocks held in registers whose every element was placed through
+// an LDS atomic of its own (62 KB of code, 300 bytes of frame); RD 2 and 4 within 0.9 us of 3.
+// All threads; ends with a barrier that hands L.big over: a block staged next clears it before a barrier of its own
+// (load_processed), and a wave still testing the last bitmaps would take masked and processed tokens' raw values.
 template <int DT>
 __device__ __noinline__ void rescan_fast(QWS_L ResolveLds* s, char* ws_, int row_, int rb_) {
   using BL = Blk<DT, NT2>;
@@ -533,108 +533,122 @@ __device__ __noinline__ void rescan_fast(QWS_L ResolveLds* s, char* ws_, int row
   const qws_row& R = S.R;
   RS& st = *L.st;
   char* const ws = uniform_ptr(ws_);
-  const int row = __builtin_amdgcn_readfirstlane(row_), rb = __builtin_amdgcn_readfirstlane(rb_);
-  const int G = __builtin_amdgcn_readfirstlane(st.G), tid = threadIdx.x;
-  unsigned long long mn = ~0ull, mx = 0ull;
-  // blocks whose processed tokens are all recorded as patches: raw logits straight into registers, RB blocks at once
-  // (all their loads in flight together); only the bin's elements are weighed, each placed at its block's next
-  // slot.  Masked and processed tokens are marked in a bitmap per block (in L.big) that the raw values found are
-  // tested against, and the patches' values are tested themselves.  (Through the staged block, one at a time, a
-  // block costs ~5 us: rows that missed 20-30 blocks took 75-150 us in all.)
-  constexpr int RB = 8;  // the resolver runs one workgroup per CU: registers for eight blocks of loads in flight
-  constexpr int BW32 = BLK / 32;
-  static_assert(RB * BW32 <= BIGW && NT2 == 2 * BW32 && TCAP == 2 * NT2, "bitmap words and patches per thread");
+  const int row = __builtin_amdgcn_readfirstlane(row_);
+  const int G = __builtin_amdgcn_readfirstlane(st.G), V = __builtin_amdgcn_readfirstlane(B.V), tid = threadIdx.x, lane = lane_id();
+  constexpr int RD = 3, BW32 = BLK / 32, GRP = 32;
+  static_assert(GRP * BW32 + GRP <= BIGW && MAXG <= 2 * GRP, "bitmaps of a group of blocks and their numbers");
   uint32_t* const bm = L.big;
-  const uint32_t flip = R.mask_mode == QWS_MASK_ALLOWED ? 0xFFFFFFFFu : 0u;
-  const unsigned* const mrow = B.masks + (R.mask_mode ? (size_t)R.mask_row * (size_t)B.mask_words : 0);
-  const int qb = st.row_top - rb;  // the bin's floor(t) >> 4
-  const float K = st.K;
-  const XRange xr = bin_xrange(qb, K);
-  auto place = [&](BI& b, int g, int local, float v) {  // the value v of block g's token, when it lies in the bin
-    const float t = tval(v, K);
-    if (v == v && v != -INFINITY && (tfloor(t) >> 4) == qb) {  // NaN counts as -inf
-      const int p = b.gofs + atomicAdd(&b.goff, 1);
-      const uint64_t c = comp(okey(v), (uint32_t)(g * BLK + local));
-      mn = c < mn ? c : mn;
-      mx = c > mx ? c : mx;
-      if (p < XG) {  // always: the bin words count these elements
-        L.ec[p] = c;
-        L.em[p] = weigh(t, L.ts).mu;
-      }
-    }
-  };
-  unsigned long long fm = readlane<unsigned long long>(st.gfast, 0);  // in scalar registers: the batches branch on it
-  while (fm) {
-    int gb[RB];
-#pragma unroll
-    for (int k = 0; k < RB; k++) {
-      gb[k] = fm ? __ffsll((long long)fm) - 1 : -1;
-      fm &= fm - 1ull;
-    }
-    // every load issued before any is used; an unused slot loads nothing (one CU reads a block at ~16 bytes per cycle)
-    float x[RB][BL::EPT];
-#pragma unroll
-    for (int k = 0; k < RB; k++) {
-      if (gb[k] >= 0) BL::load_raw(B, row, gb[k] * BLK, min(B.V, gb[k] * BLK + BLK), x[k]);  // uniform; -inf past V
-    }
-    bool marks = R.mask_mode != 0;  // uniform
-#pragma unroll
-    for (int k = 0; k < RB; k++) marks = marks || (gb[k] >= 0 && L.bi[gb[k]].n_patch > 0);
+  int* const gl = (int*)(L.big + GRP * BW32);  // the group's blocks
+  const float xlo = st.xlo, xhi = st.xhi;
+  auto hit = [&](float v) { return v >= xlo && v < xhi; };
+  unsigned long long fm = readlane<unsigned long long>(st.gfast, 0);  // in scalar registers: the loops branch on it
+  const bool marks = R.mask_mode != 0 || __ballot(lane < G && ((fm >> lane) & 1ull) && L.bi[lane].n_patch > 0) != 0ull;  // uniform
+  while (fm) {  // uniform; a group of at most GRP blocks, the lowest first
+    unsigned long long gm = fm;
+    if (__popcll(gm) > GRP) gm &= 0xFFFFFFFFull;  // MAXG <= 64: each half holds at most GRP
+    fm &= ~gm;
+    const unsigned long long gm0 = gm;
     if (marks) {
-      const int hw = tid / BW32, wi = tid % BW32;
-      uint32_t mv[RB / 2];
-#pragma unroll
-      for (int k = 0; k < RB / 2; k++) {
-        const int gk = hw ? gb[2 * k + 1] : gb[2 * k], i = gk * BW32 + wi;
-        mv[k] = R.mask_mode && gk >= 0 && i * 32 < B.V ? gmem(mrow)[i] ^ flip : 0u;
-      }
-      bar();  // the bitmaps of the batch before are read no more
-#pragma unroll
-      for (int k = 0; k < RB / 2; k++) bm[(2 * k + hw) * BW32 + wi] = mv[k];
+      const int nb = __popcll(gm);
+      bar();  // the bitmaps of the group before are read no more
+      if (tid < 64 && ((gm >> lane) & 1ull)) gl[__popcll(gm & ((1ull << lane) - 1ull))] = lane;
       bar();
-      for (int i = tid; i < TCAP; i += NT2) {  // two rounds of patches at most, the blocks' loads of a round together
-        unsigned long long pv[RB];
-        bool more = false;
+      const uint32_t flip = R.mask_mode == QWS_MASK_ALLOWED ? 0xFFFFFFFFu : 0u;
+      const unsigned* const mrow = B.masks + (R.mask_mode ? (size_t)R.mask_row * (size_t)B.mask_words : 0);
+#pragma unroll 4
+      for (int i = tid; i < nb * BW32; i += NT2) {
+        const int w = gl[i / BW32] * BW32 + i % BW32;
+        bm[i] = R.mask_mode && w * 32 < V ? gmem(mrow)[w] ^ flip : 0u;
+      }
+      bar();
+      for (int j = wave_id(); j < nb; j += NWV2) {  // a wave per block's patches
+        const int g = gl[j], np = L.bi[g].n_patch;
+        const QWS_G unsigned long long* PT = gmem((const unsigned long long*)(rec_of(ws, G, row, g) + PATCH_OFF));
+        for (int i0 = lane; i0 < np; i0 += 256) {
+          unsigned long long pv[4];
 #pragma unroll
-        for (int k = 0; k < RB; k++) {
-          const int np = gb[k] >= 0 ? L.bi[gb[k]].n_patch : 0;
-          more = more || np > NT2;
-          pv[k] = i < np ? gmem((const unsigned long long*)(rec_of(ws, G, row, max(gb[k], 0)) + PATCH_OFF))[i] : 0xFFFFFFFFull;  // local ~0: none
-        }
+          for (int k = 0; k < 4; k++) pv[k] = i0 + 64 * k < np ? PT[i0 + 64 * k] : 0xFFFFFFFFull;  // {local index, value}; local ~0: none
 #pragma unroll
-        for (int k = 0; k < RB; k++) {
-          const uint32_t l = (uint32_t)pv[k];
-          if (l != 0xFFFFFFFFu) {
-            atomicOr(&bm[k * BW32 + (l >> 5)], 1u << (l & 31));
+          for (int k = 0; k < 4; k++) {
+            const uint32_t l = (uint32_t)pv[k];
+            if (l == 0xFFFFFFFFu) continue;
+            atomicOr(&bm[j * BW32 + (l >> 5)], 1u << (l & 31));
             const float v = __uint_as_float((uint32_t)(pv[k] >> 32));
-            if (xr.maybe(v)) place(L.bi[gb[k]], gb[k], (int)l, v);
+            if (hit(v)) {
+              const int p = L.bi[g].gofs + atomicAdd(&L.bi[g].goff, 1);
+              if (p < XG) L.ec[p] = comp(okey(v), (uint32_t)g * BLK + l);  // always: the bin words count these elements
+            }
           }
         }
-        if (!more) break;  // uniform
       }
       bar();
     }
+    typename BL::Raw raw[RD];
+    float xr[RD][BL::EPT];  // bf16 blocks stay packed in raw
+    int gq[RD];
+    auto next = [&](int d) {  // the next block's loads issued
+      gq[d] = gm ? __ffsll((long long)gm) - 1 : -1;
+      gm &= gm - 1ull;
+      if (gq[d] >= 0) BL::load_bits(B, row, gq[d] * BLK, min(V, gq[d] * BLK + BLK), raw[d], xr[d]);  // uniform; -inf past V
+    };
 #pragma unroll
-    for (int k = 0; k < RB; k++) {
-      if (gb[k] < 0) continue;
-      BI& b = L.bi[gb[k]];
+    for (int d = 0; d < RD; d++) next(d);
+    while (gq[0] >= 0) {  // uniform
 #pragma unroll
-      for (int e = 0; e < BL::EPT; e++) {
-        const float v = x[k][e];
-        if (!xr.maybe(v)) continue;  // NaN fails it too
-        const int l = BL::local(e);
-        if (marks && ((bm[k * BW32 + (l >> 5)] >> (l & 31)) & 1u)) continue;
-        place(b, gb[k], l, v);
+      for (int d = 0; d < RD; d++) {
+        const int g = gq[d];
+        if (g < 0) break;  // uniform
+        float x[BL::EPT];
+        if constexpr (DT == QWS_DTYPE_F32) {
+#pragma unroll
+          for (int e = 0; e < BL::EPT; e++) x[e] = xr[d][e];
+        } else {
+          BL::unpack(raw[d], x);
+        }
+        uint32_t hm = 0;  // bit e: element e lies in the bin
+#pragma unroll
+        for (int e = 0; e < BL::EPT; e++) hm |= hit(x[e]) ? 1u << e : 0u;
+        if (marks) {
+          const uint32_t* const bg = bm + __popcll(gm0 & ((1ull << g) - 1ull)) * BW32;
+#pragma unroll
+          for (int t = 0; t < BL::S; t++) {  // a stripe's VEC tokens share a bitmap word
+            const int l = BL::local(t * BL::VEC);
+            hm &= ~(((bg[l >> 5] >> (l & 31)) & ((1u << BL::VEC) - 1u)) << (t * BL::VEC));
+          }
+        }
+        const int c = __popc(hm), inc = wave_scan_incl<int>(c), tot = readlane<int>(inc, 63);
+        if (tot) {  // uniform in the wave
+          int base = 0;
+          if (lane == 63) base = atomicAdd(&L.bi[g].goff, tot);
+          int p = L.bi[g].gofs + readlane<int>(base, 63) + inc - c;
+#pragma unroll
+          for (int e = 0; e < BL::EPT; e++) {
+            if ((hm >> e) & 1u) {
+              if (p < XG) L.ec[p] = comp(okey(x[e]), (uint32_t)(g * BLK + BL::local(e)));  // always, as above
+              p++;
+            }
+          }
+        }
+        next(d);
       }
     }
+  }
+  bar();  // every comp is there (and the bitmaps in L.big are read no more)
+  const int i1 = min(st.si[7], XG);  // the rescanned blocks' slots: behind the listed ones
+  unsigned long long mn = ~0ull, mx = 0ull;
+  for (int i = st.gl + tid; i < i1; i += NT2) {
+    const uint64_t c = L.ec[i];
+    L.em[i] = mu_of_comp(c, st.K, L.ts);
+    mn = c < mn ? c : mn;
+    mx = c > mx ? c : mx;
   }
   mn = wave_min_u64(mn);
   mx = wave_max_u64(mx);
-  if (lane_id() == 0) {
+  if (lane == 0) {
     atomicMin(&st.gmin, mn);
     atomicMax(&st.gmax, mx);
   }
-  bar();  // the bitmaps in L.big are read no more
+  bar();  // st.si[7] is read no more
 }
 
 // Gathers row bin rb (its power's fine bins staged): each block's elements come from its list when its window held
@@ -662,6 +676,14 @@ __device__ __forceinline__ void gather(ResolveLds& S, char* ws, int row, int rb)
       ln = b.gsrc == 1 ? cn : 0u;
       fr = b.gsrc == 2 && b.n_patch >= 0 ? cn : 0u;
       nres = b.gsrc == 2 ? 1 : 0;
+    }
+    if (__ballot(fr != 0) != 0ull) {  // uniform in the wave
+      float xlo = 0.0f, xhi = 0.0f;
+      if (!bin_edges(st.row_top - rb, st.K, &xlo, &xhi)) fr = 0;  // through the staged block
+      if (tid == 0) {
+        st.xlo = xlo;
+        st.xhi = xhi;
+      }
     }
     const uint32_t linc = wave_scan_incl<uint32_t>(ln), finc = wave_scan_incl<uint32_t>(fr);
     const uint32_t tot = wave_sum<uint32_t>(cn), nl = readlane<uint32_t>(linc, 63);
