@@ -1,6 +1,7 @@
 """Verify rows whose kept set is listed (at most 64 tokens: the residual drawn from the list, without the blocks) beside
-rows whose set is not, against verify_seq: set sizes around 64, both k_vfin widths of a batch's sequences mixed, draft
-probabilities that leave no residual, NaN and zero ones, the broken-residual control."""
+rows whose set is not, against verify_seq: set sizes around 64, 12 sequences of four blocks (1,024-thread verify kernels) and
+300 of one block (512-thread ones), draft probabilities that leave no residual, NaN and zero ones, the broken-residual
+control."""
 import pytest
 import torch
 
@@ -11,9 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("top_k", [1, 2, 63, 64, 65])
-def test_listed_kept_sets(top_k, dtype):
-    B, K, V, Vd = 12, 5, 3 * 8192 + 64, 4096
+@pytest.mark.parametrize("top_k,B,K,V,Vd", [*((k, 12, 5, 3 * 8192 + 64, 4096) for k in (1, 2, 63, 64, 65)), (63, 300, 2, 1024, 600)])
+def test_listed_kept_sets(top_k, B, K, V, Vd, dtype):
     tl, dp, idmap, drafts, g = _case(top_k, B, K, V, Vd, dtype, agree=0.8, noise=0.7)
     dp[1] = 0.0
     dp[2] = float("nan")
