@@ -19,8 +19,8 @@ struct Blk {
   __device__ static inline int local(int e) { return ((e / VEC) * NTH + (int)threadIdx.x) * VEC + (e % VEC); }
 
   // A block's logits on the way into x: fp32 logits are loaded there; bf16 logits stay packed (two per word) until
-  // unpack, so that a block waits for its processors' lists in half the registers (unpacked at the load, the
-  // 64-register kernel spilled the mask words behind every load: 32 rows with masks, k_scan 16.8 -> 15.3 us).
+  // unpack, so that a block waits for its processors' lists in half the registers: the 64-register k_scan spills 2 of
+  // them (8 bytes per lane), unpacked at the load 7 (28 bytes).  32 rows with masks, k_scan 16.8 -> 15.3 us.
   struct Raw {
     vu4 v[DT == QWS_DTYPE_F32 ? 1 : S];
   };

@@ -14,7 +14,8 @@ from .sampling import ValidationError
 
 
 class HeadSelect:
-    """Keeps the workspace (qws_head_ws_bytes) of one device."""
+    """Keeps the workspace (qws_head_ws_bytes) of one device: one stream at a time, as a Sampler.  The candidates and exact
+    logits it returns are views of it, valid until the next call."""
 
     def __init__(self, device="cuda"):
         self.lib = _lib.load()

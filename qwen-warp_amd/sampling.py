@@ -495,7 +495,10 @@ class ProcState:
 
 class Sampler:
     """Batched sampling stage: B rows of logits [B, V] (fp32 or bf16, on the GPU) -> B tokens.
-    One qws_sample call (two kernel launches) on the current stream; the workspace is kept per shape."""
+    One qws_sample call (two kernel launches) on the current stream; the workspace is kept per shape.  So a Sampler belongs to
+    one stream at a time: calls of one shape on two streams, or a replayed graph beside them, would write one workspace at
+    once.  Order them on the device (events, wait_stream), or use a Sampler per stream, thread or graph: sample and draft_pick
+    return without waiting for the device."""
 
     def __init__(self, device="cuda"):
         self.lib = _lib.load()
