@@ -78,6 +78,10 @@ __device__ inline bool bw_listed(unsigned long long w) { return (w >> 62) & 1ull
 // 80 bf16 verify rows, top-k 50, 46.6 / 22.2 -> 31.0 / 12.7 us; one fp32 row, top-k 20, 10.4 / 14.0 -> 8.4 / 8.0 us.
 // Larger K keeps the general records: its candidates no longer fit one wave, and the bound's overshoot grows with K.
 constexpr int TOPK_MAX = 64;                                  // the kept set fits one wave
+// A bound is accepted once at most TOP_SLACK keys more than top_k reach it: the resolver's bisection without slack (top_k 64
+// and at most 64 keys) ran through most of the 64 bits, 40 bf16 rows 17.0 -> 13.5 us.  A block's list keeps to 64 threads:
+// with 72 it exceeds TOPN more often and is cut by a second bisection (40 rows, N(0, 3) 20.6 -> 22.0 us, tied values 24 -> 52).
+constexpr int TOP_SLACK = 8;
 constexpr int TOPN = (int)(HDR_BYTES - 64) / 6;               // 74
 constexpr int TOP_KEYS = 64, TOP_IDS = TOP_KEYS + TOPN * 4;   // byte offsets of u32 okey[TOPN] and u16 local[TOPN]
 static_assert(TOP_IDS + TOPN * 2 <= (int)HDR_BYTES && TOPN >= TOPK_MAX, "top list inside the header");
@@ -1501,7 +1505,6 @@ __device__ __forceinline__ int finish_ranked(const TopRow& A, int n, const uint6
 }
 template <bool VER>
 __device__ __forceinline__ int resolve_top_body(const TopRow& A, const char* hdrs, const float2* ts, TopBuf& L) {
-  constexpr int SLACK = 8;  // entries past top_k accepted by a bound
   const int tid = threadIdx.x, lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(wave_id());
   const int K = A.K, G = A.G;
   // 2^sh threads per block: every thread holds a few entries, spread over as many threads as there are
@@ -1528,12 +1531,14 @@ __device__ __forceinline__ int resolve_top_body(const TopRow& A, const char* hdr
     int cn;
 #pragma unroll
     for (int j = 0; j < NT2 / 64; j++) m[j] = L.mxs[j * 64 + lane];
-    const uint64_t b = top_bound<NT2 / 64, uint64_t>([&](int j) { return m[j]; }, 1ull, K, min(K + SLACK, 64), &cn);
+    const uint64_t b = top_bound<NT2 / 64, uint64_t>([&](int j) { return m[j]; }, 1ull, K, G <= 32 ? K + TOP_SLACK : min(K + TOP_SLACK, 64), &cn);
     if (lane == 0) L.bound = b;
   }
   bar();
   {
-    const uint64_t b = L.bound;  // at most 64 threads hold entries at or above it
+    // at most 64 threads hold entries at or above it, or 72 of at most five each (16 threads or more per block)
+    static_assert((TOPK_MAX + TOP_SLACK) * ((TOPN + 15) / 16) <= 64 * TOP_EPL, "entries at or above the bound");
+    const uint64_t b = L.bound;
 #pragma unroll
     for (int k = 0; k < TOP_EPL; k++)
       if (c[k] >= b) L.lst[atomicAdd(&L.cnt, 1)] = c[k];

@@ -32,7 +32,7 @@ template <int DT, int NT1>
 __device__ __forceinline__ void list_top(const float (&x)[Blk<DT, NT1>::EPT], int lo, int topk, float* lmax, char* area, uint32_t* red, float* s_tv, int* s_tie,
                                          int* s_n, char* rec) {
   using BL = Blk<DT, NT1>;
-  constexpr int EPT = BL::EPT, NWV1 = NT1 / 64, SLACK = 8;
+  constexpr int EPT = BL::EPT, NWV1 = NT1 / 64;
   constexpr int LW_N = 64 * EPT;  // at most 64 threads hold listed elements
   static_assert(LW_N * 8 <= 18432 && TOPN >= TOPK_MAX, "the list's LDS");
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
@@ -48,9 +48,9 @@ __device__ __forceinline__ void list_top(const float (&x)[Blk<DT, NT1>::EPT], in
     int c;
 #pragma unroll
     for (int j = 0; j < NWV1; j++) k[j] = okey(lmax[j * 64 + lane]);
-    const uint32_t b = top_bound<NWV1, uint32_t>([&](int j) { return k[j]; }, KEY_NEGINF + 1u, topk, min(topk + SLACK, 64), &c);
+    const uint32_t b = top_bound<NWV1, uint32_t>([&](int j) { return k[j]; }, KEY_NEGINF + 1u, topk, min(topk + TOP_SLACK, 64), &c);
     if (lane == 0) {
-      const bool tie = c > min(topk + SLACK, 64);
+      const bool tie = c > min(topk + TOP_SLACK, 64);
       *s_tie = tie ? 1 : 0;
       *s_tv = okey_val(b);
     }

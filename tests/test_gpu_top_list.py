@@ -47,13 +47,13 @@ def test_top_list_rows(sampler, kind, V):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("blocks,crowd", [(17, 3), (31, 3), (32, 3), (33, 6), (64, 7)])
+@pytest.mark.parametrize("blocks,crowd", [(17, 3), (31, 3), (32, 3), (33, 6), (64, 7), (64, 9)])
 def test_top_list_rows_crowded_blocks(sampler, blocks, crowd, dtype):
     """The best tokens crowded into a few blocks whose lists are held by fewer threads than top_k (16 threads per block up to
-    32 blocks, 8 past them): the resolver's bound falls below all of them, more than 128 entries reach it, and they are
-    reduced before they are ranked."""
+    32 blocks, 8 past them; nine blocks of 64: by the 72 a bound of top_k 64 accepts): the resolver's bound falls below all of
+    them, more than 128 entries reach it, and they are reduced before they are ranked."""
     V, tpb = blocks * 8192, 16 if blocks <= 32 else 8
-    assert crowd * tpb < 64 and crowd * 64 > 128
+    assert (crowd * tpb < 58 or crowd * tpb == 72) and crowd * 58 > 128
     g = torch.Generator().manual_seed(blocks)
     B = 10
     x = torch.randn(B, V, generator=g) * 2.0
@@ -62,8 +62,23 @@ def test_top_list_rows_crowded_blocks(sampler, blocks, crowd, dtype):
         for k in torch.randperm(blocks, generator=g)[:crowd].tolist():
             x[b, k * 8192 + torch.randperm(8192, generator=g)[:300]] += 30.0
         rows.append(q.RowSpec(temperature=[1.0, 8.0][b % 2], top_k=[64, 58, 64, 64, 60][b % 5], top_p=[1.0, 0.9][b // 2 % 2], seed=b, position=b, row_key=b))
-        assert rows[-1].top_k > crowd * tpb
     check_rows(sampler, x.to(dtype), rows, label=f"blocks={blocks}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,threads", [(2, 1024), (130, 512)])
+@pytest.mark.parametrize("hot", [63, 64, 65])
+def test_top_list_rows_whole_threads(sampler, B, threads, hot, dtype):
+    """Every element of 63, 64 (the most a block's bound accepts) or 65 threads of a scan workgroup far above all others: the
+    bound lists them all, and the list is cut to what a record holds.  Both scan widths (2 x 2 and 130 x 2 workgroups)."""
+    vec, V = 4 if dtype == torch.float32 else 8, 16384
+    g = torch.Generator().manual_seed(hot)
+    x = torch.randn(B, V, generator=g)
+    for lo in (0, 8192):
+        t = torch.arange(8192) // vec % threads  # the thread that holds each token of a block
+        x[:, lo:lo + 8192] += torch.where(torch.isin(t, torch.randperm(threads, generator=g)[:hot]), 25.0, 0.0)
+    rows = [q.RowSpec(temperature=[1.0, 4.0][b % 2], top_k=[64, 63, 20][b % 3], top_p=[1.0, 0.95][b // 2 % 2], seed=b, position=b, row_key=b) for b in range(B)]
+    check_rows(sampler, x.to(dtype), rows, dense=B == 2, label=f"hot={hot}")
 
 
 @pytest.mark.parametrize("B", [7, 40])
