@@ -25,16 +25,16 @@ constexpr int CAP = 1024;                    // elements a block may list
 // The listed window of a block with more than CAP elements above its own cuts' deepest bin.
 // top-p: a flat block's own boundary is close to the row's: MARGIN_FLAT fine bins on either side.  A peaked block (its top
 // CTOP elements carry a quarter of its mass) lists one range of as many bins as the list holds, ending MARGIN_NEAR bins or
-// CAP / 4 elements below its boundary, whichever is nearer, or from its top when that fits: the row's boundary tends to lie
+// BELOW elements below its boundary, whichever is nearer, or from its top when that fits: the row's boundary tends to lie
 // above a block's own, since the outliers of other blocks add mass at the top, but where the bins are dense it is close.
 // min-p: from the top when the cut expected in the row (from the spread of the block's G best) fits the list, else the bins
 // ending at the block's own cut; with top-p too, the top-p window instead of the latter.
 // Chosen on a CPU model over rows of 31 blocks: N(0, s) logits (s 0.5-6), N(0, 2.5) with 32 tokens 8 higher, Laplace,
 // exponential, Gumbel, t(4), uniform and Zipf ones and a 1% mixture, T 0.7-1.3, top-p 0.3-0.999, min-p 0.001-0.1 and
-// both.  Rescans of eight blocks per row, summed: 265; 340 with the range ending 31 bins below the boundary whatever
+// both.  Rescans of eight blocks per row, summed: 263 (265 with BELOW = CAP / 4); 340 with the range ending 31 bins below the boundary whatever
 // they hold and the top under every min-p; 368 with two ranges, the top 256 elements and up to 100 bins around the
 // boundary.  The rows that still miss are those whose other blocks' outliers move the cut past 1,024 elements.
-constexpr int MARGIN_FLAT = 6, MARGIN_NEAR = 31;
+constexpr int MARGIN_FLAT = 6, MARGIN_NEAR = 31, BELOW = 3 * CAP / 8;
 constexpr int CTOP = 256;
 constexpr int MAXG = 64;                     // blocks per row (V <= 524,288)
 constexpr int NR = NBIN;                     // row bins with a nonzero weight (row-relative, 0 = the top)

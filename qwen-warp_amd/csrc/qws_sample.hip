@@ -488,12 +488,12 @@ __global__ void __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(NT1 !=
           } else {
             b = min(floor_r, bp + MARGIN_NEAR);
             if (b < floor_r) nb = cnt_to(b);
-            if (nb > (uint32_t)CAP) {  // uniform: at most a quarter of the list below bp, one lane per bin
+            if (nb > (uint32_t)CAP) {  // uniform: at most BELOW of the list below bp, one lane per bin
               static_assert(MARGIN_NEAR <= 64, "one lane per bin");
               const bool in = bp + 1 + lane <= b;
               const uint32_t pre = wave_scan_incl<uint32_t>(in ? (uint32_t)(hist[bp + 1 + lane] >> 40) : 0u);
               nb = cnt_to(bp);
-              const int k = __popcll(__ballot(in && pre <= (uint32_t)CAP / 4u));
+              const int k = __popcll(__ballot(in && pre <= (uint32_t)BELOW));
               b = bp + k;
               if (k > 0) nb += readlane<uint32_t>(pre, k - 1);
             }
