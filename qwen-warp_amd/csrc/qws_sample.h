@@ -31,9 +31,10 @@ constexpr int CAP = 1024;                    // elements a block may list
 // ending at the block's own cut; with top-p too, the top-p window instead of the latter.
 // Chosen on a CPU model over rows of 31 blocks: N(0, s) logits (s 0.5-6), N(0, 2.5) with 32 tokens 8 higher, Laplace,
 // exponential, Gumbel, t(4), uniform and Zipf ones and a 1% mixture, T 0.7-1.3, top-p 0.3-0.999, min-p 0.001-0.1 and
-// both.  Rescans of eight blocks per row, summed: 263 (265 with BELOW = CAP / 4); 340 with the range ending 31 bins below the boundary whatever
-// they hold and the top under every min-p; 368 with two ranges, the top 256 elements and up to 100 bins around the
-// boundary.  The rows that still miss are those whose other blocks' outliers move the cut past 1,024 elements.
+// both.  Rescans of eight blocks per row, summed: 263 (265 with BELOW = CAP / 4); 340 with the range ending 31 bins below
+// the boundary whatever they hold and the top under every min-p; 368 with two ranges, the top 256 elements and up to 100
+// bins around the boundary.  On the GPU, 640 calls of such rows take 0.842 of the time with two ranges (k_resolve's rescans
+// and small sets included).  The rows that still miss are those whose other blocks' outliers move the cut past 1,024 elements.
 constexpr int MARGIN_FLAT = 6, MARGIN_NEAR = 31, BELOW = 3 * CAP / 8;
 constexpr int CTOP = 256;
 constexpr int MAXG = 64;                     // blocks per row (V <= 524,288)
